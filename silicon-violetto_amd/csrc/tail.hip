@@ -78,67 +78,132 @@ __device__ __forceinline__ void better(float& bv, uint32_t& bi, float v, uint32_
   }
 }
 
-// kernels.metal:1484-1501 tg_scan: ex[t] = the sum of v over threads before t, in 32 serial
-// runs of 32 then their bases in order; ex[1024] = the total.
-__device__ __forceinline__ void scan1024(float v, float* ex, float* base, uint32_t tid) {
-  ex[tid] = v;
-  __syncthreads();
-  if (tid < 32) {
-    float acc = 0.0f;
-    for (uint32_t i = 32 * tid; i < 32 * tid + 32; i++) {
-      const float x = ex[i];
-      ex[i] = acc;
-      acc += x;
-    }
-    base[tid] = acc;
+// kernels.metal:1484-1501 tg_scan: thread t's share starts at the sum of v over the threads
+// before t, in 32 serial runs of 32 then their bases in order. The runs sit 33 words apart in
+// LDS, so the 32 serial lanes read 32 different banks and half a run is in registers before its
+// dependent additions start; the bases are added by the same wave from its own registers.
+struct Scan1024 {
+  float run[SV_SAMPLE_THREADS + 32];  // [32][33]: exclusive sums inside each run
+  float base[33];                     // each run's base, then the total
+  __device__ __forceinline__ float before(uint32_t t) const {
+    return t == SV_SAMPLE_THREADS ? base[32] : run[t + t / 32] + base[t / 32];
   }
-  __syncthreads();
-  if (tid == 0) {
-    float acc = 0.0f;
-    for (uint32_t g = 0; g < 32; g++) {
-      const float x = base[g];
-      base[g] = acc;
-      acc += x;
+  // Ends with a barrier; the caller has one between its last read of a scan and the next.
+  __device__ __forceinline__ void scan(float v, uint32_t tid) {
+    run[tid + tid / 32] = v;
+    __syncthreads();
+    if (tid < 64) {
+      float acc = 0.0f;
+      if (tid < 32) {
+        for (uint32_t h = 0; h < 32; h += 16) {
+          float x[16];
+#pragma unroll
+          for (int i = 0; i < 16; i++) x[i] = run[33 * tid + h + i];
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            run[33 * tid + h + i] = acc;
+            acc += x[i];
+          }
+        }
+      }
+      float b = 0.0f, mine = 0.0f;
+#pragma unroll
+      for (int g = 0; g < 32; g++) {
+        mine = tid == (uint32_t)g ? b : mine;
+        b += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), g));
+      }
+      if (tid < 32) base[tid] = mine;
+      if (tid == 0) base[32] = b;
     }
-    ex[SV_SAMPLE_THREADS] = acc;
+    __syncthreads();
   }
-  __syncthreads();
-  ex[tid] += base[tid / 32];
-  __syncthreads();
+};
+
+// sv_exp2 of an argument that is never above 0 (x - max over a positive temperature; NaN, from
+// infinite logits, gives 0 as there): the same bits without the overflow test.
+__device__ __forceinline__ float exp2_le0(float x) {
+  const float nf = __builtin_rintf(x);
+  const float f = x - nf;
+  float p = 1.525273380405984e-05f;
+  p = __builtin_fmaf(p, f, 1.5403530393381608e-04f);
+  p = __builtin_fmaf(p, f, 1.3333558146428443e-03f);
+  p = __builtin_fmaf(p, f, 9.6181291076284772e-03f);
+  p = __builtin_fmaf(p, f, 5.5504108664821580e-02f);
+  p = __builtin_fmaf(p, f, 2.4022650695910071e-01f);
+  p = __builtin_fmaf(p, f, 6.9314718055994531e-01f);
+  p = __builtin_fmaf(p, f, 1.0f);
+  return x >= -125.0f ? __builtin_amdgcn_ldexpf(p, (int)nf) : 0.0f;
 }
 
 // sample (kernels.metal:1503-1576), with argmax_partial (:1430-1451) folded in: one
 // workgroup of 1024 per row. Thread t owns ids t, t + 1024, ...: the order of every sum.
+//
+// One compute unit serves a row, so a row's passes are bound by its loads' latency and, at a
+// temperature, by the exponentials' VALU work (15 instructions an id: 15 us of 151680). Every
+// pass takes the ids past the cached ones in batches of BATCH loads, and a drawn share's ids are
+// evaluated by a whole wave at once with only their additions serial. MI355X, 32 rows of 151680
+// ids at T 0.6, top-p 0.95: 72 us (172 with one load at a time, a walk by one thread and the
+// scan's runs on two LDS banks); one greedy row 14 us (49); 5 greedy rows of 32000 4.8 us (7.1).
 __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const sv_sample_row* rows, uint32_t* out,
                                                       const uint32_t* meta, uint32_t vocab) {
-  __shared__ float ex[SV_SAMPLE_THREADS + 1];
-  __shared__ float base[32];
+  __shared__ Scan1024 sc;
   __shared__ float bvs[16];
   __shared__ uint32_t bis[16];
-  __shared__ uint32_t pick;
+  __shared__ uint32_t owner, pick;
+  __shared__ float pick_x;
+  constexpr uint32_t TOPS = 8;
+  __shared__ float top[TOPS][SV_SAMPLE_THREADS];
   const uint32_t r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const sv_sample_row row = rows[r];
   const uint32_t pos = row.tok == SV_NO_TOK ? row.pos : meta[2 * row.tok + 1] + 1;
   const float* x = logits + (size_t)r * vocab;
 
   // The first SAMPLE_CACHED logits of this thread (ids tid, tid + 1024, ...) are requested
-  // together and kept in registers (one memory round trip, and the temperature pass below
-  // reuses them); ids past that are read in the loop.
-  constexpr int SAMPLE_CACHED = 32;
+  // together and kept in registers; ids past that are read BATCH at a time. Every load is
+  // unconditional: one lane offset, a scalar one per load, and past the vocabulary the buffer's
+  // range check, whose zeros become -inf, which no pass counts.
+  constexpr int SAMPLE_CACHED = 32, BATCH = 16;
+  constexpr uint32_t NT = SV_SAMPLE_THREADS, REST = SAMPLE_CACHED * NT;
+  const float ninf = -__builtin_inff();
+  // id i0 + k of the row, i0 (below the vocabulary) the same for every lane, k < 64 Ki
+  auto at = [&](uint32_t i0, uint32_t k) {
+    const uint32_t left = min(vocab - i0, 1u << 20);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + i0), 0, left * 4, 0x00020000);
+    const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, k * 4, 0, 0));
+    return k < left ? v : ninf;
+  };
   float xc[SAMPLE_CACHED];
 #pragma unroll
-  for (int j = 0; j < SAMPLE_CACHED; j++) {
-    const uint32_t i = tid + j * SV_SAMPLE_THREADS;
-    xc[j] = i < vocab ? x[i] : 0.0f;
-  }
-  float lmax = -3.402823466e+38f;
-  uint32_t tok = 0xffffffffu;
+  for (int j = 0; j < SAMPLE_CACHED; j++) xc[j] = at(0, j * NT + tid);
+  // fn(logit, id) over the thread's BATCH ids from i0 + tid on
+  auto batch = [&](uint32_t i0, auto fn) {
+    float xb[BATCH];
 #pragma unroll
-  for (int j = 0; j < SAMPLE_CACHED; j++) {
-    const uint32_t i = tid + j * SV_SAMPLE_THREADS;
-    if (i < vocab) better(lmax, tok, xc[j], i);
+    for (int u = 0; u < BATCH; u++) xb[u] = at(i0, u * NT + tid);
+#pragma unroll
+    for (int u = 0; u < BATCH; u++) fn(xb[u], i0 + u * NT + tid);
+  };
+  // A thread's ids increase, so the first of its equal logits stands.
+  float lmax = ninf;
+  uint32_t tok = 0xffffffffu;
+  auto upper = [&](float v, uint32_t i) {
+    const bool up = v > lmax;
+    lmax = up ? v : lmax;
+    tok = up ? i : tok;
+  };
+#pragma unroll
+  for (int j = 0; j < SAMPLE_CACHED; j++) upper(xc[j], tid + j * NT);
+  // The largest logit of each of the thread's first TOPS batches, in its own LDS words: a later
+  // pass over the ids above some logit reads only the batches that hold one (a row's few likely
+  // ids leave nearly every batch unread).
+  for (uint32_t i0 = REST, b = 0; i0 < vocab; i0 += BATCH * NT, b++) {
+    float t = ninf;
+    batch(i0, [&](float v, uint32_t i) {
+      upper(v, i);
+      t = v > t ? v : t;
+    });
+    if (b < TOPS) top[b][tid] = t;
   }
-  for (uint32_t i = tid + SAMPLE_CACHED * SV_SAMPLE_THREADS; i < vocab; i += SV_SAMPLE_THREADS) better(lmax, tok, x[i], i);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const float v = __shfl_xor(lmax, o, WAVE);
@@ -152,58 +217,79 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
   __syncthreads();
   lmax = bvs[0];
   tok = bis[0];
+#pragma unroll
   for (int w = 1; w < 16; w++) better(lmax, tok, bvs[w], bis[w]);
+  if (tok == 0xffffffffu) lmax = -3.402823466e+38f;  // no id above -inf
 
   if (row.temperature > 0.0f) {
     const float c = LOG2E_F / row.temperature;
     float s = 0.0f;
+    auto add = [&](float v, uint32_t) { s += exp2_le0((v - lmax) * c); };
 #pragma unroll
-    for (int j = 0; j < SAMPLE_CACHED; j++) {
-      const uint32_t i = tid + j * SV_SAMPLE_THREADS;
-      if (i < vocab) s += sv_exp2((xc[j] - lmax) * c);
-    }
-    for (uint32_t i = tid + SAMPLE_CACHED * SV_SAMPLE_THREADS; i < vocab; i += SV_SAMPLE_THREADS)
-      s += sv_exp2((x[i] - lmax) * c);
-    scan1024(s, ex, base, tid);
-    const float z = ex[SV_SAMPLE_THREADS];
-    float low = -__builtin_inff();
+    for (int j = 0; j < SAMPLE_CACHED; j++) add(xc[j], 0);
+    for (uint32_t i0 = REST; i0 < vocab; i0 += BATCH * NT) batch(i0, add);
+    sc.scan(s, tid);
+    const float z = sc.base[32];
+    float low = ninf;
     for (uint32_t round = 0; round < SV_SAMPLE_ROUNDS; round++) {
       const u32x4 ph = philox(u32x4{pos, round, 0u, 0u}, row.seed_lo, row.seed_hi);
-      const float target = (float)(ph[0] >> 8) * 0x1p-24f * ex[SV_SAMPLE_THREADS];
-      if (tid == 0) pick = 0xffffffffu;
+      const float target = (float)(ph[0] >> 8) * 0x1p-24f * sc.base[32];
+      if (tid == 0) owner = pick = 0xffffffffu;
       __syncthreads();
-      const float lo = ex[tid];
-      if (lo <= target && target < ex[tid + 1]) {
-        // Walk this thread's ids again, summing exactly as the scan did, until the sum
-        // passes the target's offset into this thread's share. If fp32 rounding leaves the
-        // offset beyond the re-sum, the thread's last nonzero term is the pick.
-        float acc = 0.0f;
+      if (sc.before(tid) <= target && target < sc.before(tid + 1)) owner = tid;
+      __syncthreads();
+      // The owner's ids again, summed exactly as the scan did, until the sum passes the target's
+      // offset into its share: wave 0 evaluates 64 of them at a time (ids not above `low` count
+      // as 0, which no sum sees), lane l then holding the sum up to the l-th. If fp32 rounding
+      // leaves the offset beyond the re-sum, the share's last nonzero term is the pick.
+      if (wv == 0 && owner != 0xffffffffu) {
+        const uint32_t o = __builtin_amdgcn_readfirstlane(owner);
+        const float off = target - sc.before(o);
+        float acc = 0.0f, px = 0.0f;
         uint32_t j = 0xffffffffu;
-        for (uint32_t i = tid; i < vocab; i += SV_SAMPLE_THREADS) {
-          const float xi = x[i];
-          if (!(xi > low)) continue;
-          const float e = sv_exp2((xi - lmax) * c);
-          acc += e;
-          if (e > 0.0f) j = i;
-          if (target - lo < acc) break;
+        float nx = at(o, lane * NT);
+        for (uint32_t i0 = o;; i0 += 64 * NT) {
+          const float xi = nx;
+          const bool more = vocab - i0 > 64 * NT;
+          if (more) nx = at(i0 + 64 * NT, lane * NT);  // the next 64, while these are added
+          const float e = xi > low ? exp2_le0((xi - lmax) * c) : 0.0f;
+          float upto = 0.0f;
+#pragma unroll
+          for (int l = 0; l < 64; l++) {
+            acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), l));
+            upto = lane == (uint32_t)l ? acc : upto;
+          }
+          const uint64_t live = __ballot(e > 0.0f), past = __ballot(off < upto) & live;
+          if (live) {
+            const int l = past ? __builtin_ctzll(past) : 63 - __builtin_clzll(live);
+            j = i0 + l * NT;
+            px = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xi), l));
+          }
+          if (past || !more) break;
         }
-        pick = j;
+        if (lane == 0) {
+          pick = j;
+          pick_x = px;
+        }
       }
       __syncthreads();
       const uint32_t j = pick;
       if (j == 0xffffffffu) break;
-      const float xj = x[j];
+      const float xj = pick_x;
       if (xj == lmax || row.top_p >= 1.0f) {
         tok = j;
         break;
       }
       float qs = 0.0f;
-      for (uint32_t i = tid; i < vocab; i += SV_SAMPLE_THREADS) {
-        const float xi = x[i];
-        if (xi > xj) qs += sv_exp2((xi - lmax) * c);
-      }
-      scan1024(qs, ex, base, tid);
-      if (ex[SV_SAMPLE_THREADS] < row.top_p * z) {
+      auto above = [&](float v, uint32_t) {
+        if (v > xj) qs += exp2_le0((v - lmax) * c);
+      };
+#pragma unroll
+      for (int q = 0; q < SAMPLE_CACHED; q++) above(xc[q], 0);
+      for (uint32_t i0 = REST, b = 0; i0 < vocab; i0 += BATCH * NT, b++)
+        if (b >= TOPS || top[b][tid] > xj) batch(i0, above);
+      sc.scan(qs, tid);
+      if (sc.base[32] < row.top_p * z) {
         tok = j;
         break;
       }
@@ -343,12 +429,18 @@ __global__ __launch_bounds__(256) void step_tail_kernel(TailParams p) {
   __shared__ uint32_t s_k, s_len;
   const uint32_t r = blockIdx.x, tid = threadIdx.x;
   const sv_run_in ru = p.runs[r];
+  // Every row's flag first, by all threads (a prompt chunk has hundreds: one thread's stores
+  // took 12 us of a 512-row chunk's 15.5); the walk below then marks the accepted rows.
+  {
+    const uint32_t fresh = !ru.verify && !p.gen[ru.slot].done;
+    for (uint32_t j = tid; j < ru.count; j += 256) p.on_path[ru.first + j] = fresh;
+  }
+  __syncthreads();
   if (tid == 0) {
     sv_gen_state* gs = &p.gen[ru.slot];
     p.path_len[r] = 0;
     const uint32_t done = gs->done;
     uint32_t k = 0;
-    for (uint32_t j = 0; j < ru.count; j++) p.on_path[ru.first + j] = !ru.verify && !done;
     if (done) {
       p.emitted[r] = 0;
     } else {

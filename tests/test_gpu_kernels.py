@@ -493,6 +493,32 @@ def test_sample_bit_exact(gpu, vocab):
     assert np.array_equal(got, ref), f"ids differ at rows {np.nonzero(got != ref)[0]}"
 
 
+@pytest.mark.parametrize("vocab", [32768, 32769, 49152, 49153, 98305])
+def test_sample_bit_exact_past_cached(gpu, vocab):
+    """Vocabularies around the ids a thread keeps in registers (32 x 1024) and its later batches
+    (16 x 1024): trained-like rows (a few high logits, so top-p takes several rounds), and rows of
+    infinities and NaN. Bit for bit against the oracle."""
+    banner(f"sample past cached vocab={vocab}")
+    rng = np.random.default_rng(vocab)
+    n = 32
+    logits = rng.normal(14.0, 0.6, (n, vocab)).astype(np.float32)
+    for r in range(n):
+        logits[r, rng.integers(0, vocab, 12)] = rng.uniform(16, 23, 12)
+    logits[8, vocab - 1] = 23.0              # the last id of the last, partial batch
+    logits[9, :] = -np.inf
+    logits[10, rng.integers(0, vocab, 50)] = np.nan
+    logits[11, rng.integers(0, vocab, 3)] = np.inf
+    logits[12, : vocab - 3] = -np.inf
+    rows = sample_rows(n, [0.6, 0.0, 1.0, 0.05, 2.0], [0.95, 0.3, 1.0, 0.05])
+    ref = oracle.sample(L, logits, rows)
+    d_rows = torch.from_numpy(np.frombuffer(bytes((L.SampleRow * n)(*rows)), np.uint8).copy()).cuda()
+    out = torch.zeros(n, dtype=torch.int32, device="cuda")
+    K.sample(to_dev(logits), d_rows, out, None, n, vocab)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().view(np.uint32)
+    assert np.array_equal(got, ref), f"ids differ at rows {np.nonzero(got != ref)[0]}"
+
+
 # --------------------------------------------------------------- accept / compact / replay
 def random_runs(rng, n_runs, max_count=16):
     """Random verify runs over random trees, with sampled tokens that match some drafts."""
