@@ -20,8 +20,7 @@
 //     along the same path.
 // int8 weights need one scale per k chunk: groups of 256 or more, or one scale per row
 // (per-output-channel, any k).
-#include "sv_device.h"
-#include "sv_internal.h"
+#include "gemm_device.h"
 
 #include <algorithm>
 #include <mutex>
@@ -29,51 +28,9 @@
 
 namespace sv {
 
-struct MMParams {
-  const uint8_t* w;
-  const uint16_t* scales;
-  const float* x;
-  const uint32_t* x_rows;
-  float* y;
-  const float* base;
-  float* aux;
-  uint32_t n, k, m, epi, flags, vocab_real, gshift, chunks, per_row, tiled;
-  float scale, ra, rb;
-  // Split-k hand-off (skinny path with S > 1): counters per row group (zero at rest),
-  // partial sums and sums of squares per (row group, split).
-  uint32_t* counters;
-  float* part;
-  float* ssp;
-  uint32_t splits, tgroups;  // skinny: k splits and 16-token groups
-  // GEMM work order (gemm_item): 0 row block, split, token block (token block fastest); g > 0:
-  // split, groups of g row blocks, token block, row block within the group.
-  uint32_t order;
-};
-
-// The GEMMs' work item -> (token block, split, row block). Each XCD (workgroup id mod 8) takes a
-// contiguous range of items, so the order decides which weights (row block, split) and which
-// activations (token block, split) one XCD's L2 serves to several workgroups; the host picks the
-// order with the least modelled HBM traffic (gemm_order).
-__device__ __forceinline__ void gemm_item(uint32_t item, uint32_t n_tblk, uint32_t S, uint32_t nrb, uint32_t g,
-                                          uint32_t& tblk, uint32_t& sp, uint32_t& rblk) {
-  if (g == 0) {
-    tblk = item % n_tblk;
-    sp = (item / n_tblk) % S;
-    rblk = item / (n_tblk * S);
-    return;
-  }
-  const uint32_t per_sp = nrb * n_tblk, per_grp = g * n_tblk;
-  sp = item / per_sp;
-  const uint32_t rem = item % per_sp, r2 = rem % per_grp;
-  tblk = r2 / g;
-  rblk = (rem / per_grp) * g + r2 % g;
-}
-
 
 constexpr int KC = 256;  // k per chunk: one X chunk in registers, 4 blocks of 64
 constexpr int NBLK = KC / 64;
-
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 // Epilogue of the skinny kernels (kernels.metal:183-209): lane (t, q) holds rows 4 q + 0..3
 // of each of the workgroup's RT tiles for token tt; ss: the token's sum of squares over k.
@@ -656,73 +613,6 @@ __global__ __launch_bounds__(256) void pack_tiled_kernel(const uint8_t* src, uin
 //     pairs for the whole k, added in a fixed order at the end.
 //   - k splits: each split stores its sums (coherent stores) and the last split of the
 //     (row block, token block) to arrive adds them in split order and runs the epilogue.
-constexpr int GKC = 64;
-// Split-k hand-off counters (skinny and GEMM paths): a region of fixed size at the front of the
-// workspace, so every matmul sharing one workspace finds its counters at zero there, whatever
-// its shape.
-constexpr size_t COUNTER_SLOTS = 65536;
-
-// Wait for this thread's LDS operations, then the workgroup barrier. Unlike __syncthreads()
-// this leaves global loads in flight (no vmcnt wait).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Epilogue of the GEMM (kernels.metal:183-209) for one 16-token tile: lane (t16, q) holds rows
-// 4 q + 0..3 of each of the wave's RTW row tiles (first row row0) for token t.
-template <int RTW>
-__device__ __forceinline__ void gemm_epilogue(const MMParams& p, const f32x4 (&acc)[RTW], uint32_t row0, int q,
-                                              uint32_t t, float ss, bool write_inv) {
-  const float inv = 1.0f / __builtin_sqrtf(ss / (float)p.k + SV_RMS_EPS);
-  if (write_inv && (p.flags & SV_FLAG_WRITE_INV) && p.epi == SV_EPI_NORM && q == 0) p.aux[t] = inv;
-  const bool norm_in = (p.flags & SV_FLAG_NORM_IN) != 0;
-#pragma unroll
-  for (int r = 0; r < RTW; r++) {
-    const uint32_t rowq = row0 + 16 * r + 4 * q;
-    f32x4 v = acc[r];
-    const size_t o = (size_t)t * p.m + rowq;
-    switch (p.epi) {
-      case SV_EPI_NORM:
-        *(f32x4*)(p.y + o) = v * (inv * p.scale);
-        break;
-      case SV_EPI_RAW:
-        if (norm_in) v *= inv;
-        *(f32x4*)(p.y + o) = v;
-        break;
-      case SV_EPI_RESID: {
-        if (norm_in) v *= inv;
-        const f32x4 sv = v * p.scale;
-        const f32x4 b = *(const f32x4*)(p.base + o);
-        *(f32x4*)(p.y + o) = b * p.ra + sv * p.rb;
-        if (p.flags & SV_FLAG_WRITE_RAW) *(f32x4*)(p.aux + o) = sv;
-        break;
-      }
-      case SV_EPI_HEAD: {
-        if (norm_in) v *= inv;
-        f32x4 l;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          l[i] = rowq + i < p.vocab_real ? 23.0f * sigmoidf_((v[i] + 5.0f) / 7.5f) : -__builtin_inff();
-        *(f32x4*)(p.y + o) = l;
-        break;
-      }
-      case SV_EPI_SWIGLU: {
-        const float sc = inv * p.scale;
-        const float g0 = v[0] * sc, u0 = v[1] * sc, g1 = v[2] * sc, u1 = v[3] * sc;
-        float2 out;
-        out.x = g0 * sigmoidf_(g0) * u0;
-        out.y = g1 * sigmoidf_(g1) * u1;
-        *(float2*)(p.y + (size_t)t * (p.m / 2) + rowq / 2) = out;
-        break;
-      }
-      default:
-        break;
-    }
-  }
-}
-
 template <int FMT, int RTW, int NT, bool GROUPED, int GD>
 __global__ __launch_bounds__(256) void mm_gemm(MMParams p, uint32_t n_tblk) {
   static_assert(GD % 2 == 0, "chunk parity = slot parity");
@@ -993,11 +883,6 @@ __global__ __launch_bounds__(256) void mm_gemm(MMParams p, uint32_t n_tblk) {
 //     different slots mod 8 (both conflict-free on gfx950).
 //   - Lane (c, h) receives rows 8 j + 4 h + i (j, i = 0..3) of token c: f32x4 row groups, so
 //     the epilogue (rms-norm fold, SwiGLU pairs, residual) is the 16-wide one per group.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
 template <int FMT, int RT, int NT, int GD, int NW, int CPI>
 __global__ __launch_bounds__(NW * 64) void mm_gemm32(MMParams p, uint32_t n_tblk) {
   static_assert(GD % (2 * CPI) == 0, "iteration parity = buffer parity");
@@ -1294,56 +1179,84 @@ __global__ __launch_bounds__(NW * 64) void mm_gemm32(MMParams p, uint32_t n_tblk
 // S k splits.
 struct GemmCfg {
   int rtw, nt, s, d;  // d: chunks in flight (2, 4 or 8)
-  int mf = 16;        // MFMA tile: 16 (mm_gemm, tiles of 16) or 32 (mm_gemm32, tiles of 32)
+  int mf = 16;        // 16: mm_gemm (16-wide MFMA tiles), 32: mm_gemm32, 33: mm_pipe (both 32-wide)
   int nw = 4;         // waves per workgroup (mm_gemm32: 4 or 8)
   int cpi = 1;        // mm_gemm32: chunks per barrier (1, or 2 with 4 chunks in flight)
-  uint32_t bm() const { return (uint32_t)(nw * mf * rtw); }
-  uint32_t bn() const { return (uint32_t)mf * nt; }
-  uint32_t acc_bytes() const { return (uint32_t)(rtw * nt) * mf * mf / 16; }  // per thread
+  uint32_t tw() const { return mf == 16 ? 16u : 32u; }
+  uint32_t bm() const { return (uint32_t)(nw * rtw) * tw(); }
+  uint32_t bn() const { return tw() * nt; }
+  uint32_t acc_bytes() const { return (uint32_t)(rtw * nt) * tw() * tw() / 16; }  // per thread
 };
 GemmTune g_gemm_tune;  // all zero: the built-in choice
 int g_gemm_order = -1;  // tests: force a work order (-1: the modelled choice)
 
-// Built-in choice, from measurements on MI355X at 40, 160 and 512 rows (qkv, o, gate_up, down
-// int8, the bf16 head): int8 runs 32-token blocks (NT = 2) with two row tiles per wave and two
-// k splits, four when that leaves fewer than 256 workgroups; bf16 (twice the weight bytes per
-// row) runs the token block with the fewest padded tokens among NT = 3 and 5 and the fewest
-// k splits (up to 8) that give 256 workgroups. Either way one row tile per wave when the
-// splits alone cannot reach 256 workgroups, and with int8 scale groups shorter than k. At 384
-// rows and more, matrices with 512 blocks of 256 rows x 64 tokens run those (four row tiles
-// per wave, two chunks in flight), unsplit.
+// The 32 x 32-tile launch with the least modelled time (us, fitted on MI355X at 96-2048 rows with
+// the weights cold): rounds of 256 workgroups (one per compute unit), each 3.5 for its first loads
+// and its stores plus its 64-k chunks at the shape's time per chunk with the chip busy (mm_gemm32's
+// 256 x 32 block 0.55; mm_pipe's 256 x 32 0.60, 256 x 64 1.04, 512 x 32 1.10, 256 x 128 1.85,
+// 512 x 64 1.74, 512 x 128 3.2: the larger the block, the fewer operand bytes and conversions per
+// product); a split of k adds its partial sums, written and read back by the last split. The
+// blocks of 512 rows hold two sets of sums with scale groups, and spill: not offered there.
+static GemmCfg pick_tiles32(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
+  static const struct {
+    int rt, nt, cpi, mf;
+    float us, merge;  // per chunk; of the partial sums' cost, (rt nt)^0.6
+  } SHAPES[] = {{1, 1, 1, 32, 0.55f, 1.0f}, {1, 1, 2, 33, 0.60f, 1.0f}, {1, 2, 2, 33, 1.04f, 1.5f},
+                {2, 1, 1, 33, 1.10f, 1.5f}, {1, 4, 1, 33, 1.85f, 2.3f}, {2, 2, 1, 33, 1.74f, 2.3f},
+                {2, 4, 1, 33, 3.2f, 3.5f}};
+  const uint32_t nch = k / GKC;
+  GemmCfg best{1, 1, 1, 4, 33, 8, 2};
+  float best_us = 1e30f;
+  for (const auto& sh : SHAPES) {
+    if (sh.mf == 32 && (grouped || fmt != SV_FMT_I8)) continue;
+    if (grouped && sh.rt == 2 && sh.nt > 1) continue;
+    const uint32_t bm = 256u * sh.rt, bn = 32u * sh.nt;
+    if (m % bm) continue;
+    const uint64_t cells = (uint64_t)(m / bm) * ((n + bn - 1) / bn);
+    for (uint32_t s : {1u, 2u, 4u, 8u}) {
+      if (nch % s || (s > 1 && nch / s < 4)) continue;
+      const uint64_t wgs = cells * s;
+      float us = (float)((wgs + 255) / 256) * (3.5f + (nch / s) * sh.us);
+      if (s > 1) us += std::min(1.0f, wgs / 256.0f) * (2.5f + 0.8f * s) * sh.merge;
+      if (us < best_us) best_us = us, best = GemmCfg{sh.rt, sh.nt, (int)s, 4, sh.mf, 8, sh.cpi};
+    }
+  }
+  return best;
+}
+
+// Built-in choice below the 32 x 32 tiles' range (pick_tiles32), from measurements on MI355X at
+// 17-512 rows: 32-token blocks (NT = 2) of two row tiles per wave with two k splits, four when that
+// leaves fewer than 256 workgroups; one row tile per wave when the splits alone cannot reach 256
+// workgroups, and with int8 scale groups shorter than k.
 static GemmCfg pick_gemm(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   if (g_gemm_tune.rtw)
     return GemmCfg{g_gemm_tune.rtw, g_gemm_tune.nt, std::max(1, g_gemm_tune.s), g_gemm_tune.d ? g_gemm_tune.d : 4,
                    g_gemm_tune.mf ? g_gemm_tune.mf : 16, g_gemm_tune.nw ? g_gemm_tune.nw : 4,
                    g_gemm_tune.cpi ? g_gemm_tune.cpi : 1};
   const uint32_t nch = k / GKC;
-  // int8 at 96 rows and more: 32 x 32 tiles, 8 waves, four chunks in flight; one 32-row tile
-  // per wave (256-row blocks) and 32 tokens, or for the widest matrices two tiles per wave
-  // (512-row blocks) and 64 tokens from 384 rows; the fewest k splits that give 160
-  // workgroups. Measured on MI355X against the 16-wide shapes below at 160 and 512 rows: qkv
-  // 14.0 -> 13.4 and 23.6 -> 20.1 us, o 13.9 -> 13.1 and 20.5 -> 17.8, down 26.5 -> 23.9 and
-  // 51.6 -> 44.1, gate_up 34.2 -> 31.6 and 73.5 -> 67.6.
-  const bool wide = m >= 8192 && m % 512 == 0;
-  if (fmt == SV_FMT_I8 && !grouped && n >= 96 && m % 256 == 0) {
-    GemmCfg c{wide ? 2 : 1, wide && n >= 384 ? 2 : 1, 1, 4, 32, 8, 1};
-    const uint32_t cells = m / c.bm() * ((n + c.bn() - 1) / c.bn());
-    for (int s : {1, 2, 4, 8})
-      if (nch % s == 0 && nch / s >= 4) {
-        c.s = s;
-        if (cells * s >= 160) break;
-      }
-    return c;
+  const uint64_t tiles = (uint64_t)(m / 256) * ((n + 31) / 32) * nch;  // 256-row x 32-token x 64-k blocks
+  const bool big = (uint64_t)m * k * (fmt == SV_FMT_I8 ? 1 : 2) > (96ull << 20);
+  // The 32 x 32 tiles, wherever the work fills them (m a multiple of 256). Both sides measured on
+  // MI355X at 24-2048 rows, weights cold:
+  //  - int8 with a scale per row: from 96 rows (gate_up 96 rows 27.5 -> 23.1 us, 2048 rows 290 ->
+  //    213; below, the 16-wide tiles: qkv 64 rows 12.1 against 12.8);
+  //  - int8 in scale groups: from 1500 blocks (gate_up of the 1280-wide model at 512 rows 47 -> 27,
+  //    at 2048 187 -> 87, down at 256 27 -> 21; below, o at 256 rows 14.5 against 15.7);
+  //  - bf16: from 4096 blocks (gate_up 192 rows 54 -> 38, 2048 rows 337 -> 265; below, o at 256
+  //    rows 16.2 against 17.4);
+  //  - bf16 weights too large to stay cached (the 131 MB head): from 49 rows (64 rows 46 -> 39,
+  //    256 rows 113 -> 75), but two 80-token blocks at 129-160 rows (63 against 66).
+  if (m % 256 == 0) {
+    const bool wide = fmt == SV_FMT_I8 ? (grouped ? tiles >= 1500 : n >= 96)
+                      : big            ? n > 48 && (n <= 128 || n > 160)
+                                       : tiles >= 4096;
+    if (wide) return pick_tiles32(fmt, grouped, n, m, k);
   }
-  // Wide matrices at many rows: 256-row x 64-token blocks halve the operand traffic through
-  // L2 (weights re-read per token block, X per row block) where they still fill the device.
-  // Two chunks in flight (not four) keep that shape at two waves per SIMD.
-  if (!grouped && n >= 384 && m % 256 == 0 && (uint64_t)(m / 256) * ((n + 63) / 64) >= 384) return GemmCfg{4, 4, 1, 2};
   // Weights too large to stay cached between token blocks (the 131 MB bf16 head) are re-read
   // from HBM by every token block: below that shape, the fewest token blocks (48 or 80 tokens,
   // whichever pads n least), no k splits, four chunks in flight for 48 tokens (measured with
   // the weights cold: 20-25 % faster than 32-token blocks or split k at 40 and 160 rows).
-  if (!grouped && (uint64_t)m * k * (fmt == SV_FMT_I8 ? 1 : 2) > (96ull << 20)) {
+  if (!grouped && big) {
     GemmCfg c{m % 128 ? 1 : 2, 3, 1, 4};
     uint32_t best = ~0u;
     for (int nt : {3, 5}) {
@@ -1403,6 +1316,9 @@ static size_t gemm_ws_layout(uint32_t n, uint32_t m, const GemmCfg& c, size_t* s
 
 static bool gemm_shape_ok(uint32_t m, uint32_t k, const GemmCfg& c) {
   const bool nt_ok = c.nt == 2 || c.nt == 3 || c.nt == 4 || c.nt == 5 || c.nt == 8;
+  if (c.mf == 33)
+    return gemm_pipe_built(c.rtw, c.nt, c.cpi) && c.nw == 8 && c.s >= 1 && c.s <= 64 &&
+           m % c.bm() == 0 && (k / GKC) % c.s == 0;
   // 32-wide tiles: one or two row tiles per wave, one to three token tiles.
   if (c.mf == 32)
     return (c.rtw == 1 || c.rtw == 2) && c.nt >= 1 && c.nt <= 3 && (c.d == 2 || c.d == 4) && (c.nw == 4 || c.nw == 8) &&
@@ -1510,7 +1426,7 @@ static uint32_t gemm_order(uint32_t nrb, uint32_t n_tblk, uint32_t S, double w_b
 static sv_status gemm_launch(hipStream_t stream, uint32_t fmt, MMParams& p, void* ws, size_t ws_bytes) {
   const bool grouped = fmt == SV_FMT_I8 && !p.per_row;
   const GemmCfg c = pick_gemm(fmt, grouped, p.n, p.m, p.k);
-  if (!gemm_shape_ok(p.m, p.k, c) || (grouped && (c.rtw != 1 || c.mf != 16)))
+  if (!gemm_shape_ok(p.m, p.k, c) || (grouped && c.mf != 33 && (c.rtw != 1 || c.mf != 16)))
     return fail(SV_ERR_ARG, "matmul (gemm): launch shape rtw %d, nt %d, splits %d for m %u, k %u", c.rtw, c.nt, c.s,
                 p.m, p.k);
   if ((size_t)p.m * p.k * (fmt == SV_FMT_I8 ? 1 : 2) >= (1ull << 31) || (size_t)p.n * p.k * 4 >= (1ull << 31))
@@ -1534,7 +1450,9 @@ static sv_status gemm_launch(hipStream_t stream, uint32_t fmt, MMParams& p, void
                                 : gemm_order(rb, n_tblk, c.s, c.bm() * kk * (fmt == SV_FMT_I8 ? 1 : 2), c.bn() * kk * 4);
     if (p.order && rb % p.order) p.order = 0;
   }
-  if (c.mf == 32) {
+  if (c.mf == 33) {
+    gemm_pipe_launch(stream, fmt, grouped, c.rtw, c.nt, c.cpi, p, nwg, n_tblk);
+  } else if (c.mf == 32) {
     gemm_dispatch32(stream, fmt, c, p, nwg, n_tblk);
   } else if (fmt == SV_FMT_I8) {
     if (grouped) gemm_dispatch_nt<SV_FMT_I8, 1, true>(stream, p, c.nt, c.d, nwg, n_tblk);

@@ -16,7 +16,7 @@ from conftest import banner
 from helpers import bf16_bits, close, to_dev, u16_dev_bf16
 from violetto import _lib as L
 from violetto import kernels as K
-from violetto.model import ModelShape, quantize_rows
+from violetto.model import ModelShape, quantize_groups, quantize_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -791,6 +791,56 @@ def test_matmul_gemm_launch_shapes(gpu, shape, n):
                   what=f"bf16 call {call}")
     finally:
         tune[0] = tune[1] = tune[2] = tune[3] = tune[4] = tune[5] = tune[6] = 0
+
+
+@pytest.mark.parametrize("rt,nt,cpi", [(1, 1, 2), (1, 2, 2), (1, 4, 1), (2, 1, 1), (2, 2, 1), (2, 4, 1)])
+@pytest.mark.parametrize("splits", [1, 4, 8])
+@pytest.mark.parametrize("n", [17, 100, 170])
+def test_matmul_pipe_launch_shapes(gpu, rt, nt, cpi, splits, n):
+    """Every shape of mm_pipe (row tiles per wave, token tiles, chunks per iteration) with one to
+    eight k splits of odd and even chunk counts: int8 per row with gathered rows (EPI_NORM and the
+    inverse norms), int8 in groups of 64 and 128 (EPI_SWIGLU), bf16 (EPI_RESID), row-major and
+    tiled, over ragged token blocks; two calls share one workspace."""
+    banner(f"pipe rt={rt} nt={nt} cpi={cpi} splits={splits} n={n}")
+    tune = (C.c_int * 7).in_dll(L.lib(), "_ZN2sv11g_gemm_tuneE")
+    rng = np.random.default_rng(rt * 1000 + nt * 100 + splits * 10 + n)
+    m, k = 512 * rt, 2560 if splits == 8 else 1280  # 20 chunks; five in each of 4 or 8 splits
+    ws = K.Workspace(64 << 20)
+    w = torch.from_numpy(rng.normal(0, 0.02, (m, k)).astype(np.float32))
+    x = (rng.normal(0, 1, (n + 3, k)) * rng.uniform(0.5, 4, (n + 3, 1))).astype(np.float32)
+    rows = rng.permutation(n + 3)[:n].astype(np.uint32)
+    base = rng.normal(0, 1, (n, m)).astype(np.float32)
+    bits = lambda t: t.view(torch.int16).numpy().view(np.uint16)  # noqa: E731
+
+    def check(mat, host_w, host_s, gs, epi, x_in, what, flags=0, x_rows=None, b=None):
+        a = L.MatArgs(n, k, m, epi, flags, m, 0.75, 1.1, 0.7, 1, k, gs)
+        aux_ref = np.zeros(n, np.float32)
+        ref = oracle.matmul(L, host_w, host_s, gs, x_in, a, base=b, aux=aux_ref, x_rows=x_rows)
+        y = torch.zeros(n, m // 2 if epi == L.EPI_SWIGLU else m, device="cuda")
+        aux = torch.zeros(n, device="cuda")
+        K.matmul(mat, to_dev(x_in), y, n=n, epi=epi, flags=flags, scale=0.75, ra=1.1, rb=0.7, aux=aux,
+                 base=None if b is None else to_dev(b), x_rows=None if x_rows is None else to_dev(x_rows), ws=ws)
+        torch.cuda.synchronize()
+        close(y.cpu().numpy(), ref, atol=5e-5 * max(float(np.abs(ref).max()), 1.0), rtol=1e-4, what=what)
+        if flags & L.FLAG_WRITE_INV:
+            close(aux.cpu().numpy(), aux_ref, atol=1e-5, rtol=1e-4, what=f"{what} inv")
+
+    try:
+        for i, v in enumerate((rt, nt, splits, 4, 33, 8, cpi)):
+            tune[i] = v
+        q, s = quantize_rows(w)
+        check(K.matrix(q.cuda(), s.cuda(), 31), q.numpy(), bits(s), 31, L.EPI_NORM, x, "per row",
+              L.FLAG_WRITE_INV, rows)
+        for g in (64, 128):
+            q, s = quantize_groups(w, g)
+            gs = g.bit_length() - 1
+            mat = K.matrix(q.cuda(), s.cuda(), gs)
+            check(mat.tiled() if g == 64 else mat, q.numpy(), bits(s), gs, L.EPI_SWIGLU, x[:n].copy(), f"groups of {g}")
+        wb = bf16_bits(w.numpy())
+        check(K.matrix(u16_dev_bf16(wb)).tiled(), wb, None, 0, L.EPI_RESID, x[:n].copy(), "bf16", b=base)
+    finally:
+        for i in range(7):
+            tune[i] = 0
 
 
 def test_matmul_skinny_groups_of_256(gpu):
