@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "layers.h"
@@ -351,10 +352,18 @@ struct sv_engine {
   // device: one step set (plan.rs writes these per step)
   // tokens: the plan's ids (FEED_ROW + i kept, so a captured step can be replayed); tok_res:
   // the ids embed resolved, which accept compares.
+  // All but tok_res lie in one block, packed by each plan (upload_plan) and copied at once from its
+  // pinned twin.
   uint32_t *tokens = nullptr, *tok_res = nullptr, *tin = nullptr, *vis = nullptr, *head_rows = nullptr,
            *attn_runs = nullptr;
   sv_sample_row* sample_rows = nullptr;
   sv_run_in* runs = nullptr;
+  uint8_t *plan_dev = nullptr, *plan_host = nullptr;
+  size_t plan_cap = 0;
+  // Pinned memory a step's outputs are read back through (sv_step): emitted and ids, then logits.
+  uint8_t* back = nullptr;
+  size_t back_ids = 0, back_logits = 0;  // bytes of each part
+  uint32_t* host_table = nullptr;        // pinned twin of the page table
   uint32_t *out_ids = nullptr, *emitted = nullptr, *meta = nullptr, *path = nullptr, *path_len = nullptr,
            *on_path = nullptr;
   // device: activations (buffers.rs Scratch)
@@ -422,8 +431,8 @@ struct sv_engine {
 
   ~sv_engine() {
     if (graph) (void)hipGraphExecDestroy(graph);
-    void* bufs[] = {k_cache, v_cache, page_table, rope, rope_rows, lens, feed, tree, trace, trace_len, gen, tokens, tok_res, tin, vis,
-                    head_rows, attn_runs, sample_rows, runs, out_ids, emitted, meta, path, path_len, on_path, h, qkv,
+    void* bufs[] = {k_cache, v_cache, page_table, rope, rope_rows, lens, feed, tree, trace, trace_len, gen, tok_res, plan_dev,
+                    emitted, meta, path, path_len, on_path, h, qkv,
                     attn, mixed, act, inv, logits, ws, mm_ws, k_local, v_local, local_table, h0, xattn, rbase, vdir};
     for (void* b : bufs)
       if (b) (void)hipFree(b);
@@ -431,6 +440,8 @@ struct sv_engine {
       if (b) (void)hipFree(b);
     for (void* b : {(void*)pl_buf, (void*)pl_sync})
       if (b) (void)hipFree(b);
+    for (void* b : {(void*)plan_host, (void*)back, (void*)host_table})
+      if (b) (void)hipHostFree(b);
     if (head_tiled) (void)hipFree(head_tiled);
     if (head_lo_tiled) (void)hipFree(head_lo_tiled);
     if (tap[0]) (void)hipFree(tap[0]);
@@ -474,8 +485,9 @@ struct sv_engine {
   float* emb_out() const { return extras.n_mudd ? h0 : h; }
   float* in_of(uint32_t li) const { return li == 0 ? emb_out() : out_of(li - 1); }
 
-  // kv.rs:49-56 reserve(): pages until the slot holds `len` positions; the page table
-  // entry goes to the device at once.
+  // kv.rs:49-56 reserve(): pages until the slot holds `len` positions; the page table entries go to
+  // the device from pinned memory. The caller has waited for the stream before (an earlier copy may
+  // still read the same rows) and waits for it, or launches the step behind it, afterwards.
   sv_status reserve(uint32_t slot, uint32_t len) {
     auto& pg = pages[slot];
     const size_t before = pg.size();
@@ -486,10 +498,10 @@ struct sv_engine {
       free_pages.pop_back();
     }
     if (pg.size() > before) {
-      SV_HIP(hipMemcpyAsync(page_table + (size_t)slot * max_pages + before, pg.data() + before,
-                            (pg.size() - before) * 4, hipMemcpyHostToDevice, stream),
-             "page table");
-      SV_HIP(hipStreamSynchronize(stream), "page table");
+      // (the stream is idle: no earlier copy still reads the pinned rows)
+      const size_t at = (size_t)slot * max_pages + before, words = pg.size() - before;
+      memcpy(host_table + at, pg.data() + before, words * 4);
+      SV_HIP(hipMemcpyAsync(page_table + at, host_table + at, words * 4, hipMemcpyHostToDevice, stream), "page table");
     }
     return SV_OK;
   }
@@ -517,6 +529,31 @@ struct sv_engine {
     SV_HIP(hipMalloc(&mm_ws, bytes), "matmul workspace");
     SV_HIP(hipMemset(mm_ws, 0, bytes), "matmul workspace");
     mm_ws_bytes = bytes;
+    return SV_OK;
+  }
+
+  // A plan's arrays packed into the pinned block and copied in one piece (seven copies from pageable
+  // memory took about 20 us of a step's host time). The samples come last: sv_sample_logits may write
+  // as many rows as the block was made for.
+  sv_status upload_plan(const std::vector<uint32_t>& tok, const std::vector<uint32_t>& ti, const std::vector<uint32_t>& vi,
+                        const std::vector<uint32_t>& hr, const std::vector<uint32_t>& ar,
+                        const std::vector<sv_run_in>& ri, const std::vector<sv_sample_row>& sr) {
+    size_t off = 0;
+    auto put = [&](const void* src, size_t bytes, auto** ptr) {
+      off = (off + 15) / 16 * 16;
+      *ptr = reinterpret_cast<std::remove_reference_t<decltype(*ptr)>>(plan_dev + off);
+      if (off + bytes <= plan_cap && bytes) memcpy(plan_host + off, src, bytes);
+      off += bytes;
+    };
+    put(tok.data(), tok.size() * 4, &tokens);
+    put(ti.data(), ti.size() * 4, &tin);
+    put(vi.data(), vi.size() * 4, &vis);
+    put(hr.data(), hr.size() * 4, &head_rows);
+    put(ar.data(), ar.size() * 4, &attn_runs);
+    put(ri.data(), ri.size() * sizeof(sv_run_in), &runs);
+    put(sr.data(), sr.size() * sizeof(sv_sample_row), &sample_rows);
+    if (off > plan_cap) return fail(SV_ERR_CAPACITY, "plan: %zu bytes of step arrays (%zu)", off, plan_cap);
+    SV_HIP(hipMemcpyAsync(plan_dev, plan_host, off, hipMemcpyHostToDevice, stream), "plan upload");
     return SV_OK;
   }
 
@@ -1022,16 +1059,15 @@ extern "C" sv_status sv_engine_create(const sv_engine_config* cfg, const float* 
   ALLOC(trace, (size_t)S * cfg->max_seq_len);
   ALLOC(trace_len, S);
   ALLOC(gen, S);
-  ALLOC(tokens, n);
   ALLOC(tok_res, n);
-  ALLOC(tin, 2 * (size_t)n);
-  ALLOC(vis, n);
-  ALLOC(head_rows, n);
-  ALLOC(attn_runs, 2 * ((size_t)n / e->arun + S));
-  ALLOC(sample_rows, std::max(n, R));
-  ALLOC(runs, S);
-  ALLOC(out_ids, std::max(n, R));
-  ALLOC(emitted, S);
+  // the emitted counts and, 64 words on at least, the ids: one copy reads both back
+  const size_t em_words = ((size_t)S + 63) / 64 * 64;
+  ALLOC(emitted, em_words + std::max(n, R));
+  e->out_ids = e->emitted + em_words;
+  e->plan_cap = 7 * 16 + (size_t)n * 20 + ((size_t)n / e->arun + S) * 8 + S * sizeof(sv_run_in) +
+                (size_t)std::max(n, R) * sizeof(sv_sample_row);
+  ALLOC(plan_dev, e->plan_cap);
+  e->sample_rows = (sv_sample_row*)e->plan_dev;
   ALLOC(meta, 2 * (size_t)n);
   ALLOC(rope_rows, (size_t)n * SV_ROPE_PAIRS * 2);
   ALLOC(path, (size_t)S * SV_FEED_W);
@@ -1045,6 +1081,14 @@ extern "C" sv_status sv_engine_create(const sv_engine_config* cfg, const float* 
   ALLOC(inv, n);
   ALLOC(logits, (size_t)std::max(n, R) * s.vocab);
 #undef ALLOC
+  // Pinned: the plan's block, the outputs (logits of up to 1 MB; larger ones go straight to the
+  // caller's memory) and the page table's twin.
+  e->back_ids = (em_words + std::max(n, R)) * 4;
+  e->back_logits = std::min((size_t)std::max(n, R) * s.vocab * 4, (size_t)1 << 20);
+  if (hipHostMalloc((void**)&e->plan_host, e->plan_cap, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&e->back, e->back_ids + e->back_logits, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&e->host_table, (size_t)S * e->max_pages * 4, hipHostMallocDefault) != hipSuccess)
+    return bad(fail(SV_ERR_HIP, "pinned step buffers"));
   // RoPE table (engine.rs:394-421): (bf16(cos), bf16(sin)) of float(pos) * freq[j].
   {
     const size_t npos = (size_t)cfg->max_seq_len + SV_FEED_W;
@@ -1474,13 +1518,7 @@ extern "C" sv_status sv_new_seq(sv_engine* e, uint32_t* slot) {
   e->seq_len[s] = 0;
   e->pages[s].clear();
   e->sampling[s] = sv_sample_row{0, 0, 0, 0.0f, 1.0f, SV_NO_TOK};
-  const uint32_t zero = 0;
-  sv_gen_state g;
-  memset(&g, 0, sizeof g);
-  g.remaining = 0xffffffffu;
-  SV_TRY(e->upload(e->lens + s, &zero, 4));
-  SV_TRY(e->upload(e->trace_len + s, &zero, 4));
-  SV_TRY(e->upload(e->gen + s, &g, sizeof g));
+  SV_TRY(seq_init_launch(e->stream, e->lens + s, e->trace_len + s, e->gen + s));
   SV_HIP(hipStreamSynchronize(e->stream), "new_seq");
   *slot = s;
   return SV_OK;
@@ -1537,6 +1575,7 @@ extern "C" sv_status sv_bench_fill(sv_engine* e, uint32_t slot, uint32_t len) {
   SV_TRY(check_slot(e, slot));
   const uint64_t nl = (uint64_t)e->seq_len[slot] + len;
   if (nl > e->cfg.max_seq_len) return fail(SV_ERR_CAPACITY, "sequence would reach %llu tokens", (unsigned long long)nl);
+  SV_HIP(hipStreamSynchronize(e->stream), "bench_fill");
   SV_TRY(e->reserve(slot, (uint32_t)nl));
   e->seq_len[slot] = (uint32_t)nl;
   const uint32_t v = (uint32_t)nl;
@@ -1556,6 +1595,7 @@ extern "C" sv_status sv_set_feed(sv_engine* e, uint32_t slot, uint32_t len, uint
   SV_TRY(check_slot(e, slot));
   if (len > e->cfg.max_seq_len) return fail(SV_ERR_CAPACITY, "set_feed: length %u", len);
   if (token >= e->sh.vocab) return fail(SV_ERR_ARG, "set_feed: token %u", token);
+  SV_HIP(hipStreamSynchronize(e->stream), "set_feed");
   SV_TRY(e->reserve(slot, len));
   e->seq_len[slot] = len;
   SV_TRY(e->upload(e->lens + slot, &len, 4));
@@ -1571,9 +1611,10 @@ extern "C" sv_status sv_set_replay(sv_engine* e, uint32_t seed, float rate) {
   return SV_OK;
 }
 
-// plan.rs:47-151 Engine::plan.
-extern "C" sv_status sv_plan(sv_engine* e, const sv_run* runs_in, uint32_t n_runs, uint32_t extra_keys,
-                             sv_plan_info* info) {
+// plan.rs:47-151 Engine::plan. The copies are left in the stream, ahead of the step (sv_plan waits
+// for them, sv_step for the whole step).
+static sv_status make_plan(sv_engine* e, const sv_run* runs_in, uint32_t n_runs, uint32_t extra_keys,
+                           sv_plan_info* info) {
   if (!e || (!runs_in && n_runs)) return fail(SV_ERR_ARG, "plan: null pointer");
   if (n_runs == 0) return fail(SV_ERR_ARG, "plan: no runs");
   if (n_runs > e->cfg.max_seqs) return fail(SV_ERR_CAPACITY, "plan: %u runs", n_runs);
@@ -1731,15 +1772,10 @@ extern "C" sv_status sv_plan(sv_engine* e, const sv_run* runs_in, uint32_t n_run
     SV_TRY(e->upload(e->d_vis, dvis.data(), dvis.size() * 4));
     SV_TRY(e->upload(e->d_tiles, dtiles.data(), dtiles.size() * 4));
   }
-  SV_TRY(e->upload(e->tokens, tokens.data(), tokens.size() * 4));
-  SV_TRY(e->upload(e->tin, tin.data(), tin.size() * 4));
-  SV_TRY(e->upload(e->vis, vis.data(), vis.size() * 4));
-  SV_TRY(e->upload(e->head_rows, head_rows.data(), head_rows.size() * 4));
-  SV_TRY(e->upload(e->sample_rows, samples.data(), samples.size() * sizeof(sv_sample_row)));
-  SV_TRY(e->upload(e->runs, run_in.data(), run_in.size() * sizeof(sv_run_in)));
-  SV_TRY(e->upload(e->attn_runs, attn_runs.data(), attn_runs.size() * 4));
+  e->planned = false;  // the arrays of an earlier plan end here
+  SV_TRY(e->upload_plan(tokens, tin, vis, head_rows, attn_runs, run_in, samples));
   SV_TRY(e->plan_layers(P));
-  SV_HIP(hipStreamSynchronize(e->stream), "plan upload");
+  if (P.n_blocks || P.persist) SV_HIP(hipStreamSynchronize(e->stream), "plan upload");  // copied from this frame's vectors
   e->plan = P;
   e->planned = true;
   if (info) {
@@ -1751,6 +1787,13 @@ extern "C" sv_status sv_plan(sv_engine* e, const sv_run* runs_in, uint32_t n_run
     info->split = P.split;
     info->max_splits = P.max_splits;
   }
+  return SV_OK;
+}
+
+extern "C" sv_status sv_plan(sv_engine* e, const sv_run* runs, uint32_t n_runs, uint32_t extra_keys,
+                             sv_plan_info* info) {
+  SV_TRY(make_plan(e, runs, n_runs, extra_keys, info));
+  SV_HIP(hipStreamSynchronize(e->stream), "plan upload");
   return SV_OK;
 }
 
@@ -1805,13 +1848,18 @@ static sv_status step_planned(sv_engine* e, const sv_run* runs, uint32_t n_runs,
                               float* logits, uint32_t* emitted, const sv_plan_info& pi) {
   SV_TRY(e->issue(1));
   SV_TRY(e->encode(flags));
+  // The outputs come back through pinned memory, queued behind the step: one wait for all of them.
+  const size_t em_words = e->out_ids - e->emitted, lg = logits ? (size_t)pi.n_head * e->sh.vocab * 4 : 0;
+  SV_HIP(hipMemcpyAsync(e->back, e->emitted, (pi.n_head ? em_words + pi.n_head : n_runs) * 4, hipMemcpyDeviceToHost, e->stream),
+         "step ids");
+  if (lg && lg <= e->back_logits)
+    SV_HIP(hipMemcpyAsync(e->back + e->back_ids, e->logits, lg, hipMemcpyDeviceToHost, e->stream), "step logits");
   SV_HIP(hipStreamSynchronize(e->stream), "step");
   SV_TRY(e->check_layers());
-  std::vector<uint32_t> em(n_runs);
-  SV_HIP(hipMemcpy(em.data(), e->emitted, n_runs * 4, hipMemcpyDeviceToHost), "step emitted");
-  if (ids && pi.n_head) SV_HIP(hipMemcpy(ids, e->out_ids, pi.n_head * 4, hipMemcpyDeviceToHost), "step ids");
-  if (logits && pi.n_head)
-    SV_HIP(hipMemcpy(logits, e->logits, (size_t)pi.n_head * e->sh.vocab * 4, hipMemcpyDeviceToHost), "step logits");
+  std::vector<uint32_t> em((const uint32_t*)e->back, (const uint32_t*)e->back + n_runs);
+  if (ids && pi.n_head) memcpy(ids, (const uint32_t*)e->back + em_words, pi.n_head * 4);
+  if (lg && lg <= e->back_logits) memcpy(logits, e->back + e->back_ids, lg);
+  else if (lg) SV_HIP(hipMemcpy(logits, e->logits, lg, hipMemcpyDeviceToHost), "step logits");
   if (emitted) memcpy(emitted, em.data(), n_runs * 4);
   for (uint32_t ri = 0; ri < n_runs; ri++)
     if (runs[ri].verify) {
@@ -1824,7 +1872,7 @@ static sv_status step_planned(sv_engine* e, const sv_run* runs, uint32_t n_runs,
 extern "C" sv_status sv_step(sv_engine* e, const sv_run* runs, uint32_t n_runs, uint32_t flags, uint32_t* ids,
                              float* logits, uint32_t* emitted, sv_plan_info* info) {
   sv_plan_info pi;
-  SV_TRY(sv_plan(e, runs, n_runs, 0, &pi));
+  SV_TRY(make_plan(e, runs, n_runs, 0, &pi));
   if (info) *info = pi;
   return step_planned(e, runs, n_runs, flags, ids, logits, emitted, pi);
 }
@@ -1836,7 +1884,7 @@ extern "C" sv_status sv_step_capture(sv_engine* e, const sv_run* runs, uint32_t 
                                      sv_plan_info* info) {
   if (!e || !fn) return fail(SV_ERR_ARG, "step_capture: null engine or callback");
   sv_plan_info pi;
-  SV_TRY(sv_plan(e, runs, n_runs, 0, &pi));
+  SV_TRY(make_plan(e, runs, n_runs, 0, &pi));
   if (info) *info = pi;
   const uint32_t n = e->plan.n, H = e->sh.hidden, NQD = e->sh.n_heads * e->sh.head_dim;
   const uint32_t NKD = e->sh.n_kv_heads * e->sh.head_dim;

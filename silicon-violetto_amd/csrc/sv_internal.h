@@ -136,6 +136,8 @@ sv_status draft_conv_launch(hipStream_t stream, const float* x, const float* cor
 sv_status mudd_launch(hipStream_t stream, const float* cur, const float* tap0, const float* tap1, const float* dense1,
                       const float* mix, float* out_attn, float* out_base, uint32_t n, uint32_t hidden);
 
+sv_status seq_init_launch(hipStream_t stream, uint32_t* len, uint32_t* trace_len, sv_gen_state* gen);
+
 // A paged K/V cache kv_compact moves rows in: n_layers layers of n_pages pages through `table`.
 struct KvCacheRef {
   uint16_t* kc;

@@ -832,6 +832,22 @@ sv_status replay_launch(hipStream_t stream, const sv_run_in* runs, uint32_t nrun
 
 namespace sv {
 
+// A new sequence's device state: length and trace 0, an open budget without stop ids.
+__global__ __launch_bounds__(64) void seq_init_kernel(uint32_t* len, uint32_t* trace_len, uint32_t* gen) {
+  const uint32_t i = threadIdx.x;
+  if (i == 0) *len = *trace_len = 0;
+  if (i < sizeof(sv_gen_state) / 4) gen[i] = i == offsetof(sv_gen_state, remaining) / 4 ? 0xffffffffu : 0u;
+}
+
+sv_status seq_init_launch(hipStream_t stream, uint32_t* len, uint32_t* trace_len, sv_gen_state* gen) {
+  launch(seq_init_kernel, dim3(1), dim3(64), 0, stream, len, trace_len, (uint32_t*)gen);
+  return check_launch("new_seq");
+}
+
+}  // namespace sv
+
+namespace sv {
+
 sv_status step_tail_launch(hipStream_t stream, const sv_shape* sh, const sv_run_in* runs, uint32_t nruns,
                            const uint32_t* tokens, uint32_t* out, uint32_t* lens, uint32_t* feed, sv_gen_state* gen,
                            uint32_t* emitted, uint32_t* tree, uint32_t* path, uint32_t* path_len, uint32_t* on_path,
