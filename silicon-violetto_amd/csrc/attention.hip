@@ -148,23 +148,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     // Rope words through a descriptor whose range is empty without rope (zeros, no access), so
     // no branch splits the loads' accounting. Inline runs: the step's rows by token, in this
     // same round trip; else the table's rows at the positions, once those are in.
-    float2 cs[NCT][KST][4];
+    float2 cs[NCT][ROPE_KS][4];
     auto load_rope = [&](const float* base, bool by_token) {
       const __amdgpu_buffer_rsrc_t rrs =
           __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, p.rope_on ? 0x7fffffff : 0, 0x00020000);
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-        for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-          for (int jj = 0; jj < 4; jj++) {
-            const uint32_t j = 16 * ks + 4 * q + jj;
-            const bool on = p.rope_on && 32 * ks + 8 * q < 64;
-            const uint32_t c = min(16u * ct + c16, ncols - 1);
-            const uint32_t row = by_token ? t0 + c / p.G : qr.pos[ct];
-            const uint32_t off = (row * SV_ROPE_PAIRS + j) * 8 + (on ? 0u : 0x80000000u);
-            cs[ct][ks][jj] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rrs, off, 0, 0));
-          }
+      for (int ct = 0; ct < NCT; ct++) {
+        const uint32_t c = min(16u * ct + c16, ncols - 1);
+        rope_words(rrs, by_token ? t0 + c / p.G : qr.pos[ct], cs[ct], q);
+      }
     };
     if constexpr (INL) load_rope(p.rope_rows, true);
     __builtin_amdgcn_sched_barrier(0);
@@ -210,15 +202,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     }
     __builtin_amdgcn_sched_barrier(0);
     if (tid < T) svis[tid] = visw;
-    // 3. The queries, while the batches stream (columns past the run's are zero; no rope is
-    //    the identity rotation).
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-      for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++)
-          if (!(p.rope_on && 32 * ks + 8 * q < 64)) cs[ct][ks][jj] = float2{1.0f, 0.0f};
+    // 3. The queries, while the batches stream (columns past the run's are zero).
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++)
       if (16u * ct + c16 >= ncols)
@@ -326,11 +310,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     l += __shfl_xor(l, 16, WAVE);
     l += __shfl_xor(l, 32, WAVE);
     const uint32_t col = 16 * ct + c16;
-    float* od = ored + ((size_t)wv * COLS + col) * D;
+    f32x4* od = (f32x4*)ored + ((size_t)wv * COLS + col) * (D / 4);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int dt = 0; dt < VE; dt++) od[16 * dt + 4 * q + i] = O[dt][ct][i];
+    for (int dt = 0; dt < VE; dt++) od[red_slot<D>(c16, 4 * dt + q)] = O[dt][ct];
     if (q == 0) lred[wv * COLS + col] = l;
   }
   __syncthreads();
@@ -339,9 +321,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
   {
     const __amdgpu_buffer_rsrc_t po = coherent_rsrc(p.part_o + rec * p.maxcols * D);
     for (uint32_t i4 = tid; i4 < n4; i4 += 256) {
-      const f32x4* o4 = (const f32x4*)ored;
-      const uint32_t cs = COLS * D / 4;
-      store_wt4(po, i4 * 16, ((o4[i4] + o4[cs + i4]) + o4[2 * cs + i4]) + o4[3 * cs + i4]);
+      const uint32_t col = i4 / (D / 4);
+      const f32x4* o4 = (const f32x4*)ored + col * (D / 4) + red_slot<D>(col, i4 % (D / 4));
+      constexpr uint32_t cs = COLS * D / 4;
+      store_wt4(po, i4 * 16, ((o4[0] + o4[cs]) + o4[2 * cs]) + o4[3 * cs]);
     }
   }
   float* pl = p.part_l + rec * p.maxcols;
@@ -571,23 +554,12 @@ __global__ __launch_bounds__(256) void attn_capture_kernel(AttnParams p) {
         }
       }
     }
-    float2 cs[NCT][KST][4];
+    float2 cs[NCT][ROPE_KS][4];
     const __amdgpu_buffer_rsrc_t rrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(INL ? p.rope_rows : p.rope), 0, p.rope_on ? 0x7fffffff : 0, 0x00020000);
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-      for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-          const uint32_t j = 16 * ks + 4 * q + jj;
-          const bool on = p.rope_on && 32 * ks + 8 * q < 64;
-          const uint32_t c = min(16u * ct + c16, ncols - 1);
-          const uint32_t row = INL ? t0 + c / p.G : qr.pos[ct];
-          const uint32_t off = (row * SV_ROPE_PAIRS + j) * 8 + (on ? 0u : 0x80000000u);
-          cs[ct][ks][jj] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rrs, off, 0, 0));
-          if (!on) cs[ct][ks][jj] = float2{1.0f, 0.0f};
-        }
+      rope_words(rrs, INL ? t0 + min(16u * ct + c16, ncols - 1) / p.G : qr.pos[ct], cs[ct], q);
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++)
       if (16u * ct + c16 >= ncols)

@@ -121,158 +121,6 @@ __device__ __forceinline__ size_t readlane64(size_t v, int l) {
   return ((size_t)hi << 32) | lo;
 }
 
-template <int VE>
-struct VWord;
-template <>
-struct VWord<4> {
-  typedef u32x2 type;
-};
-template <>
-struct VWord<8> {
-  typedef u32x4 type;
-};
-
-// One batch of 32 keys [kb, kb + 32) below kend, for one wave: its K and V words (loaded
-// ahead of use) and the products. NEW: the keys are the run's new ones, in LDS (index
-// key - p0), masked by each column's vis.
-template <int D>
-struct KvBatch {
-  static constexpr int KST = D / 32, VE = D / 16;
-  typedef typename VWord<VE>::type vword;
-  u32x4 kw[2][KST];  // lane (c16, q): key kb + 16 mt + c16, dims 32 ks + 8 q .. + 7
-  vword vw[8];       // slot j: key kb + 16 (j / 4) + 4 q + j % 4, dims VE c16 .. + VE - 1
-};
-
-// toff: the element offsets of the batch's two 16-key tiles when the caller has them (no
-// page-table load then).
-template <int D, bool NEW>
-__device__ __forceinline__ void load_batch(const AttnParams& p, uint32_t seq, uint32_t g, uint32_t kb, uint32_t kend,
-                                           uint32_t p0, const uint16_t* nk, const uint16_t* nv, KvBatch<D>& b,
-                                           int lane, const size_t* toff = nullptr) {
-  constexpr int KST = D / 32, VE = D / 16;
-  typedef typename KvBatch<D>::vword vword;
-  const int c16 = lane & 15, q = lane >> 4;
-  // A tile of 16 keys never straddles a page (pages hold >= 16 keys, kb is a multiple of 32).
-#pragma unroll
-  for (int mt = 0; mt < 2; mt++) {
-    const uint32_t first = min(kb + 16 * mt, kend - 1);
-    const uint16_t* kt;
-    const uint16_t* vt;
-    if (NEW) {
-      kt = nk + (size_t)(first - p0) * D;
-      vt = nv + (size_t)(first - p0) * D;
-    } else {
-      const size_t off = toff ? toff[mt] : kv_off<D>(p, seq, g, first);
-      kt = p.kc + off;
-      vt = p.vc + off;
-    }
-    const uint32_t key = min(kb + 16 * mt + c16, kend - 1);
-    const uint16_t* kr = kt + (size_t)(key - first) * D;
-#pragma unroll
-    for (int ks = 0; ks < KST; ks++) b.kw[mt][ks] = *(const u32x4*)(kr + 32 * ks + 8 * q);
-#pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-      const uint32_t vk = min(kb + 16 * mt + 4 * q + jj, kend - 1);
-      b.vw[4 * mt + jj] = *(const vword*)(vt + (size_t)(vk - first) * D + VE * c16);
-    }
-  }
-}
-
-// A cached batch through per-tile buffer descriptors: its two 16-key tiles start at the
-// page-aligned positions kb and kb + 16 (toff: their element offsets, the page table applied,
-// clamped into the pool), so a tile's 16 keys lie in its page and each lane's byte offset
-// within a tile is the same for every batch: no per-key address arithmetic. Keys at or past
-// the context end are read (inside the page) and masked by compute_batch.
-template <int D>
-__device__ __forceinline__ void load_batch_tiles(const AttnParams& p, const size_t* toff, KvBatch<D>& b, int lane) {
-  constexpr int KST = D / 32, VE = D / 16;
-  typedef typename KvBatch<D>::vword vword;
-  const int c16 = lane & 15, q = lane >> 4;
-  const uint32_t ko = (uint32_t)(c16 * D + 8 * q) * 2;      // key c16, dims 8 q .. (+ 32 ks)
-  const uint32_t vo = (uint32_t)(4 * q * D + VE * c16) * 2;  // key 4 q (+ jj), dims VE c16 ..
-#pragma unroll
-  for (int mt = 0; mt < 2; mt++) {
-    const __amdgpu_buffer_rsrc_t krs = coherent_rsrc(p.kc + toff[mt]), vrs = coherent_rsrc(p.vc + toff[mt]);
-#pragma unroll
-    for (int ks = 0; ks < KST; ks++) b.kw[mt][ks] = buf_ld16(krs, ko + 64 * ks, 0);
-#pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-      if constexpr (VE == 4)
-        b.vw[4 * mt + jj] = __builtin_bit_cast(vword, __builtin_amdgcn_raw_buffer_load_b64(vrs, vo + jj * D * 2, 0, 0));
-      else
-        b.vw[4 * mt + jj] = __builtin_bit_cast(vword, buf_ld16(vrs, vo + jj * D * 2, 0));
-    }
-  }
-}
-
-// FULL: every key of the batch is below kend (no key mask). Columns past ncols need no mask
-// either: their queries are zero, so they only fill partial sums that are never stored.
-// p = 2^s by the hardware exp (v_exp_f32): q and k are rms-normed, so |s| <= D x scale x
-// log2 e (11.6 at D = 64, scale 1/8) and no result is subnormal.
-template <int D, int NCT, bool NEW, bool FULL = false>
-__device__ __forceinline__ void compute_batch(const AttnParams& p, const KvBatch<D>& b, uint32_t kb, uint32_t kend,
-                                              uint32_t p0, uint32_t ncols, uint32_t t0,
-                                              const bf16x8 (&qh)[NCT][D / 32], const bf16x8 (&ql)[NCT][D / 32],
-                                              f32x4 (&O)[D / 16][NCT], float (&lsum)[NCT], int lane,
-                                              const uint32_t* vis_cached = nullptr) {
-  constexpr int KST = D / 32, VE = D / 16;
-  const int c16 = lane & 15, q = lane >> 4;
-  // S^T tiles: lane holds keys kb + 16 mt + 4 q + i, column 16 ct + c16.
-  f32x4 S[2][NCT];
-#pragma unroll
-  for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++) {
-      f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KST; ks++) {
-        const bf16x8 kk = __builtin_bit_cast(bf16x8, b.kw[mt][ks]);
-        a = mfma16(kk, qh[ct][ks], a);
-        a = mfma16(kk, ql[ct][ks], a);
-      }
-      S[mt][ct] = a;
-    }
-  bf16x8 ph[NCT], pl[NCT];
-#pragma unroll
-  for (int ct = 0; ct < NCT; ct++) {
-    const uint32_t c = 16 * ct + c16;
-    const bool col_ok = c < ncols;
-    uint32_t vbits = 0;
-    if (NEW && col_ok) vbits = vis_cached ? vis_cached[c / p.G] : p.vis[t0 + c / p.G];
-    float pv[8];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t key = kb + 16 * mt + 4 * q + i;
-        float e = __builtin_amdgcn_exp2f(S[mt][ct][i]);
-        if (!FULL) {
-          bool ok = col_ok && key < kend;
-          if (NEW) ok = ok && ((vbits >> (key - p0)) & 1u);
-          e = ok ? e : 0.0f;
-        }
-        pv[4 * mt + i] = e;
-        lsum[ct] += e;
-      }
-    split8(pv, ph[ct], pl[ct]);
-  }
-  // O^T[dt] (rows: dims VE (4 q + i) + dt) += V^T[dt] P^T.
-#pragma unroll
-  for (int dt = 0; dt < VE; dt++) {
-    u32x4 a;
-    const uint32_t sel = (dt & 1) ? 0x07060302u : 0x05040100u;
-#pragma unroll
-    for (int jj = 0; jj < 4; jj++) a[jj] = __builtin_amdgcn_perm(b.vw[2 * jj + 1][dt >> 1], b.vw[2 * jj][dt >> 1], sel);
-    const bf16x8 av = __builtin_bit_cast(bf16x8, a);
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++) {
-      O[dt][ct] = mfma16(av, ph[ct], O[dt][ct]);
-      O[dt][ct] = mfma16(av, pl[ct], O[dt][ct]);
-    }
-  }
-}
-
-
 // ----------------------------------------------------------------------------------------
 // The attention kernel's batches carry V as the tile's own bytes (coalesced 16-byte loads) and
 // transpose it on the way into the matrix cores through a wave-private LDS stage with gfx950's
@@ -286,7 +134,11 @@ struct KvBatchT {
   u32x4 vr[2][NV];   // tile mt (keys kb + 16 mt ..): its bytes 16 lane + 1024 v (rows of 2 D bytes)
 };
 
-// Cached batch through per-tile buffer descriptors (load_batch_tiles' contract).
+// A cached batch through per-tile buffer descriptors: its two 16-key tiles start at the
+// page-aligned positions kb and kb + 16 (toff: their element offsets, the page table applied,
+// clamped into the pool), so a tile's 16 keys lie in its page and each lane's byte offset
+// within a tile is the same for every batch: no per-key address arithmetic. Keys at or past
+// the context end are read (inside the page) and masked by compute_batch_t.
 // oob = 2^31 turns every load into a range-checked miss: zeros, no memory access (a batch
 // slot past the split's last batch).
 template <int D>
@@ -337,8 +189,12 @@ constexpr uint32_t stage_row() { return 2 * D + 32; }
 template <int D>
 constexpr uint32_t stage_bytes() { return 32 * stage_row<D>(); }  // 2 tiles x 16 keys
 
-// compute_batch's semantics with V through the wave's LDS stage (2 tiles x 16 keys, rows of
-// stage_row bytes).
+// One batch's products, V through the wave's LDS stage (2 tiles x 16 keys, rows of stage_row
+// bytes). FULL: every key of the batch is below kend (no key mask). Columns past ncols need no
+// mask either: their queries are zero, so they only fill partial sums that are never stored.
+// NEW: the keys are the run's new ones, masked by each column's vis. p = 2^s by the hardware exp
+// (v_exp_f32): q and k are rms-normed, so |s| <= D x scale x log2 e (11.6 at D = 64, scale 1/8)
+// and no result is subnormal.
 // Keys at or past kend that a partial batch read from their page get V rows of zero, so
 // whatever the cache holds there cannot reach the sums (p is 0 for them).
 // clo: each lane column's first visible cached key (key_lo; 0 on global layers); a FULL batch
@@ -438,60 +294,35 @@ struct QRaw {
   uint32_t pos[NCT];
 };
 
-template <int D, int NCT, bool COH>
-__device__ __forceinline__ void qload(const AttnParams& p, uint32_t t0, uint32_t g, uint32_t ncols, QRaw<D, NCT>& r,
-                                      int lane) {
-  constexpr int KST = D / 32;
-  const int c16 = lane & 15, q = lane >> 4;
+// RoPE turns a head's first 64 dims: the first two steps of 32.
+constexpr int ROPE_KS = 2;
+// A column's rope words (pairs 16 ks + 4 q .. + 3) from `row` of the table or of the step's rows,
+// as 16-byte loads.
+__device__ __forceinline__ void rope_words(__amdgpu_buffer_rsrc_t rrs, uint32_t row, float2 (&cs)[ROPE_KS][4], int q) {
 #pragma unroll
-  for (int ct = 0; ct < NCT; ct++) {
-    const uint32_t c = 16 * ct + c16;
-    r.pos[ct] = 0;
-    if (c < ncols) {
-      const uint32_t i = c / p.G, h = g * p.G + c % p.G, t = t0 + i;
-      r.pos[ct] = p.meta[2 * t + 1];
-      const size_t qo = (size_t)t * p.W + h * D + 8 * q;
+  for (int ks = 0; ks < ROPE_KS; ks++)
 #pragma unroll
-      for (int ks = 0; ks < KST; ks++) {
-        const f32x4 a = ld_act<COH>(p.qkv, qo + 32 * ks), b = ld_act<COH>(p.qkv, qo + 32 * ks + 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          r.v[ct][ks][e] = a[e];
-          r.v[ct][ks][4 + e] = b[e];
-        }
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) r.v[ct][ks][e] = 0.0f;
+    for (int jj = 0; jj < 4; jj += 2) {
+      const f32x4 w = __builtin_bit_cast(f32x4, buf_ld16(rrs, (row * SV_ROPE_PAIRS + 16 * ks + 4 * q + jj) * 8, 0));
+      cs[ks][jj] = float2{w[0], w[1]};
+      cs[ks][jj + 1] = float2{w[2], w[3]};
     }
-  }
 }
 
-// The rope words of a lane's columns (all columns requested together).
-template <int D, int NCT>
-__device__ __forceinline__ void qrope_load(const AttnParams& p, uint32_t ncols, const QRaw<D, NCT>& r,
-                                           float2 (&cs)[NCT][D / 32][4], int lane) {
-  constexpr int KST = D / 32;
-  const int c16 = lane & 15, q = lane >> 4;
-#pragma unroll
-  for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-    for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-      for (int jj = 0; jj < 4; jj++) {
-        const uint32_t j = 16 * ks + 4 * q + jj;
-        const bool on = p.rope_on && 16 * ct + c16 < ncols && 32 * ks + 8 * q < 64;
-        cs[ct][ks][jj] = !on ? float2{1.0f, 0.0f} : *(const float2*)(p.rope + ((size_t)r.pos[ct] * SV_ROPE_PAIRS + j) * 2);
-      }
-}
+// Place of a column's 16-byte group ch within its row of the reduction buffer: permuted by the
+// column's low bits, so the 16 columns that a quarter wave writes fall on all banks. (Rows of D
+// words in order put the 16 columns on one bank, 16 passes per write: with the rope words in
+// 8-byte loads, also for dims without RoPE, a workgroup of 64 columns took about 19 us beside its
+// batches. Attention at 32 streams x 8 rows, D = 128: 82 -> 68 us; 32 trees of 16, D = 64: 76 -> 68;
+// one stream x 5 rows, all batches in flight: 9.6 -> 8.2.)
+template <int D>
+__device__ __forceinline__ uint32_t red_slot(uint32_t col, uint32_t ch) { return ch ^ (col & 15u); }
 
-// Norm, RoPE (words from qrope_load), scale and hi/lo split of the raw queries.
+// Norm, RoPE (words from rope_words; none: p.rope_on is 0), scale and hi/lo split of the raw queries.
 // CAP (the capture kernel only): the queries after the norm and RoPE also go to p.cap_q.
 template <int D, int NCT, bool CAP = false>
 __device__ __forceinline__ void qfinish_cs(const AttnParams& p, uint32_t ncols, QRaw<D, NCT>& r,
-                                           const float2 (&cs)[NCT][D / 32][4], bf16x8 (&qh)[NCT][D / 32],
+                                           const float2 (&cs)[NCT][ROPE_KS][4], bf16x8 (&qh)[NCT][D / 32],
                                            bf16x8 (&ql)[NCT][D / 32], int lane, uint32_t t0 = 0, uint32_t g = 0) {
   constexpr int KST = D / 32;
   const int c16 = lane & 15, q = lane >> 4;
@@ -511,7 +342,7 @@ __device__ __forceinline__ void qfinish_cs(const AttnParams& p, uint32_t ncols, 
       float* v = r.v[ct][ks];
 #pragma unroll
       for (int e = 0; e < 8; e++) v[e] *= inv;
-      if (p.rope_on && ok && 32 * ks + 8 * q < 64) {
+      if (ks < ROPE_KS && p.rope_on && ok) {
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
           const float a0 = v[2 * jj], a1 = v[2 * jj + 1];
@@ -531,26 +362,6 @@ __device__ __forceinline__ void qfinish_cs(const AttnParams& p, uint32_t ncols, 
       split8(v, qh[ct][ks], ql[ct][ks]);
     }
   }
-}
-
-template <int D, int NCT>
-__device__ __forceinline__ void qfinish(const AttnParams& p, uint32_t ncols, QRaw<D, NCT>& r, bf16x8 (&qh)[NCT][D / 32],
-                                        bf16x8 (&ql)[NCT][D / 32], int lane) {
-  float2 cs[NCT][D / 32][4];
-  qrope_load<D, NCT>(p, ncols, r, cs, lane);
-  qfinish_cs<D, NCT>(p, ncols, r, cs, qh, ql, lane);
-}
-
-// Queries of columns 16 ct + c16 (kernels.metal:1022-1039 with norm_rope :727-736): rms-norm
-// over the head, RoPE on pairs, times softmax scale x log2 e, split into bf16 hi + lo MFMA
-// operands; k slot j of step ks is dim 32 ks + 8 q + j. COH: qkv is read with coherent
-// loads (written earlier in the same launch by other workgroups).
-template <int D, int NCT, bool COH>
-__device__ __forceinline__ void build_queries(const AttnParams& p, uint32_t t0, uint32_t g, uint32_t ncols,
-                                              bf16x8 (&qh)[NCT][D / 32], bf16x8 (&ql)[NCT][D / 32], int lane) {
-  QRaw<D, NCT> r;
-  qload<D, NCT, COH>(p, t0, g, ncols, r, lane);
-  qfinish<D, NCT>(p, ncols, r, qh, ql, lane);
 }
 
 // The run's new keys (kernels.metal:910-942 new_key): norm, RoPE, bf16, to the cache at

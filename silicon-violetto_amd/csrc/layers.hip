@@ -346,7 +346,7 @@ __device__ __forceinline__ void attn_compute(const AttnParams& p, AttnItem& a, c
   }
   // queries (rope words by token: the step's rows), visibility words
   QRaw<D, NCT> qr;
-  float2 cs[NCT][KST][4];
+  float2 cs[NCT][ROPE_KS][4];
   const __amdgpu_buffer_rsrc_t rrs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.rope_rows), 0, p.rope_on ? 0x7fffffff : 0, 0x00020000);
 #pragma unroll
@@ -361,14 +361,8 @@ __device__ __forceinline__ void attn_compute(const AttnParams& p, AttnItem& a, c
         qr.v[ct][ks][e] = x0[e];
         qr.v[ct][ks][4 + e] = x1[e];
       }
-#pragma unroll
-      for (int jj = 0; jj < 4; jj++) {
-        const uint32_t jp = 16 * ks + 4 * q + jj;
-        const bool on = p.rope_on && 32 * ks + 8 * q < 64;
-        const uint32_t off = (t * SV_ROPE_PAIRS + jp) * 8 + (on ? 0u : 0x80000000u);
-        cs[ct][ks][jj] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rrs, off, 0, 0));
-      }
     }
+    rope_words(rrs, t, cs[ct], q);
   }
   const uint32_t visw = p.vis[t0 + min((uint32_t)tid, T - 1)];
   if ((uint32_t)tid < T) svis[tid] = visw;
@@ -378,13 +372,6 @@ __device__ __forceinline__ void attn_compute(const AttnParams& p, AttnItem& a, c
     asm volatile("" : "+v"(q0));
     rec[6] = __builtin_amdgcn_s_memrealtime() + (q0 == 12345.0f ? 1 : 0);
   }
-#pragma unroll
-  for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-    for (int ks = 0; ks < KST; ks++)
-#pragma unroll
-      for (int jj = 0; jj < 4; jj++)
-        if (!(p.rope_on && 32 * ks + 8 * q < 64)) cs[ct][ks][jj] = float2{1.0f, 0.0f};
 #pragma unroll
   for (int ct = 0; ct < NCT; ct++)
     if (16u * ct + c16 >= ncols)
@@ -438,11 +425,9 @@ __device__ __forceinline__ void attn_compute(const AttnParams& p, AttnItem& a, c
     l += __shfl_xor(l, 16, WAVE);
     l += __shfl_xor(l, 32, WAVE);
     const uint32_t col = 16 * ct + c16;
-    float* od = ored + ((size_t)wv * COLS + col) * D;
+    f32x4* od = (f32x4*)ored + ((size_t)wv * COLS + col) * (D / 4);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int dt = 0; dt < VE; dt++) od[16 * dt + 4 * q + i] = O[dt][ct][i];
+    for (int dt = 0; dt < VE; dt++) od[red_slot<D>(c16, 4 * dt + q)] = O[dt][ct];
     if (q == 0) lred[wv * COLS + col] = l;
   }
   __syncthreads();
@@ -450,10 +435,11 @@ __device__ __forceinline__ void attn_compute(const AttnParams& p, AttnItem& a, c
   const size_t rec_i = ((size_t)a.r * p.NKV + g) * p.max_splits + s;
   const uint32_t n4 = ncols * D / 4;
   const __amdgpu_buffer_rsrc_t po = coherent_rsrc(p.part_o + rec_i * p.maxcols * D);
-  const uint32_t cs4 = COLS * D / 4;
+  constexpr uint32_t cs4 = COLS * D / 4;
   for (uint32_t i4 = tid; i4 < n4; i4 += 256) {
-    const f32x4* o4 = (const f32x4*)ored;
-    store_wt4(po, i4 * 16, ((o4[i4] + o4[cs4 + i4]) + o4[2 * cs4 + i4]) + o4[3 * cs4 + i4]);
+    const uint32_t col = i4 / (D / 4);
+    const f32x4* o4 = (const f32x4*)ored + col * (D / 4) + red_slot<D>(col, i4 % (D / 4));
+    store_wt4(po, i4 * 16, ((o4[0] + o4[cs4]) + o4[2 * cs4]) + o4[3 * cs4]);
   }
   float* pl = p.part_l + rec_i * p.maxcols;
   for (uint32_t idx = tid; idx < ncols; idx += 256)
