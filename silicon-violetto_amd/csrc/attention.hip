@@ -61,6 +61,15 @@ constexpr int attn_waves(int D, int, int) { return D == 64 ? 2 : 1; }
 // workgroup adds parallelism: the trees 2 % faster).
 constexpr bool attn_newest_own(int NCT, int NBW) { return NBW > 0 || NCT >= 3; }
 
+// Whether the four waves share the query build (wave w builds column tile w, LDS exchanges them): the
+// norm, RoPE and split of a tile are about 1300 cycles of vector work at D = 128, and its words 12 loads,
+// against a round trip through LDS behind the barrier that is there anyway. Attention kernel before and
+// after, D = 128: 32 streams x 8 rows (three tiles) 68 -> 52 us, a 512-token chunk's window layers (four
+// tiles; its 43 runs also inline) 28 -> 24, global layers 76 -> 71; D = 64: 32 trees of 16 rows (four)
+// 68 -> 61, 32 streams x 5 rows (two) 68 -> 65.5. One tile has nothing to share, and the all-in-flight
+// variant's waves build their two while the batches are on their way.
+constexpr bool attn_share_queries(int NCT, int NBW) { return NBW == 0 && NCT >= 2; }
+
 // NBW = 0: each wave keeps one batch in flight ahead of the one it multiplies (any split).
 // NBW > 0 (splits of at most 128 NBW keys, grids of about one workgroup per CU): each wave
 // requests all of its batches at once, after the queries, positions and page-table words (one
@@ -117,7 +126,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
   const uint32_t nbw_full = p.split / 32 > (uint32_t)wv ? (p.split / 32 - wv + 3) / 4 : 0u;
   size_t tile_off = 0;
   const uint32_t ncols = T * p.G;
+  // Shared build: wave w takes columns cb .. cb + 15 (its queries are exchanged behind the V stages).
+  constexpr bool SHARE = attn_share_queries(NCT, NBW);
+  constexpr int QT = SHARE ? 1 : NCT;
+  const uint32_t cb = SHARE ? 16u * wv : 0u, qcols = ncols > cb ? ncols - cb : 0u;
   bf16x8 qh[NCT][KST], ql[NCT][KST];
+  u32x4* qx = (u32x4*)((char*)lds + 4 * stage_bytes<D>());  // [NCT][KST][hi, lo][lane]
   KvBatchT<D> bt[NBW > 0 ? NBW : 1];
   {
     // Queries, positions and page-table words in one round trip; then the rope words, then
@@ -126,10 +140,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     // 1. One round trip: query words and positions of the lane's columns (a column past the
     //    run's reads the last column's words and is zeroed), this wave's page-table words
     //    (lane 2 i + mt: tile mt of batch i, index clamped into the table) and p0.
-    QRaw<D, NCT> qr;
+    QRaw<D, QT> qr;
 #pragma unroll
-    for (int ct = 0; ct < NCT; ct++) {
-      const uint32_t c = min(16u * ct + c16, ncols - 1), i = c / p.G, h = g * p.G + c % p.G, t = t0 + i;
+    for (int ct = 0; ct < QT; ct++) {
+      const uint32_t c = min(cb + 16u * ct + c16, ncols - 1), i = c / p.G, h = g * p.G + c % p.G, t = t0 + i;
       qr.pos[ct] = p.meta[2 * t + 1];
       const size_t qo = (size_t)t * p.W + h * D + 8 * q;
 #pragma unroll
@@ -148,13 +162,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     // Rope words through a descriptor whose range is empty without rope (zeros, no access), so
     // no branch splits the loads' accounting. Inline runs: the step's rows by token, in this
     // same round trip; else the table's rows at the positions, once those are in.
-    float2 cs[NCT][ROPE_KS][4];
+    float2 cs[QT][ROPE_KS][4];
     auto load_rope = [&](const float* base, bool by_token) {
       const __amdgpu_buffer_rsrc_t rrs =
           __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, p.rope_on ? 0x7fffffff : 0, 0x00020000);
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) {
-        const uint32_t c = min(16u * ct + c16, ncols - 1);
+      for (int ct = 0; ct < QT; ct++) {
+        const uint32_t c = min(cb + 16u * ct + c16, ncols - 1);
         rope_words(rrs, by_token ? t0 + c / p.G : qr.pos[ct], cs[ct], q);
       }
     };
@@ -204,13 +218,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     if (tid < T) svis[tid] = visw;
     // 3. The queries, while the batches stream (columns past the run's are zero).
 #pragma unroll
-    for (int ct = 0; ct < NCT; ct++)
-      if (16u * ct + c16 >= ncols)
+    for (int ct = 0; ct < QT; ct++)
+      if (16u * ct + c16 >= qcols)
 #pragma unroll
         for (int ks = 0; ks < KST; ks++)
 #pragma unroll
           for (int e = 0; e < 8; e++) qr.v[ct][ks][e] = 0.0f;
-    qfinish_cs<D, NCT>(p, ncols, qr, cs, qh, ql, lane);
+    if constexpr (SHARE) {
+      bf16x8 th[1][KST], tl[1][KST];
+      qfinish_cs<D, 1>(p, qcols, qr, cs, th, tl, lane);
+      if (wv < NCT)
+#pragma unroll
+        for (int ks = 0; ks < KST; ks++) {
+          qx[((wv * KST + ks) * 2) * WAVE + lane] = __builtin_bit_cast(u32x4, th[0][ks]);
+          qx[((wv * KST + ks) * 2 + 1) * WAVE + lane] = __builtin_bit_cast(u32x4, tl[0][ks]);
+        }
+    } else {
+      qfinish_cs<D, NCT>(p, ncols, qr, cs, qh, ql, lane);
+    }
   }
 
   const uint32_t nsplit = attn_nsplit_t<LOCAL>(p, p0);
@@ -245,6 +270,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
 
   if (newest) new_keys<D, false>(p, seq, g, t0, T, p0, nk, nv, tid, 256);
   __syncthreads();
+  if constexpr (SHARE) {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
+      for (int ks = 0; ks < KST; ks++) {
+        qh[ct][ks] = __builtin_bit_cast(bf16x8, qx[((ct * KST + ks) * 2) * WAVE + lane]);
+        ql[ct][ks] = __builtin_bit_cast(bf16x8, qx[((ct * KST + ks) * 2 + 1) * WAVE + lane]);
+      }
+  }
 
   f32x4 O[VE][NCT];
   float lsum[NCT];
@@ -719,7 +753,8 @@ sv_status attn_launch(hipStream_t stream, const sv_shape* sh, const float* qkv, 
   }
   if (parts & 1) {
     dim3 grid(args->max_splits, NKV, n_runs);
-    // the reduction buffer, at least the 4 waves' V stages (2 x 16 rows of 2 D + 32 bytes) it holds
+    // the reduction buffer, at least the 4 waves' V stages (2 x 16 rows of 2 D + 32 bytes) it holds (from
+    // two column tiles on it is larger than the stages and the 4 maxcols D bytes of queries behind them)
     const size_t shm = std::max((size_t)4 * maxcols * D * 4 + (size_t)4 * maxcols * 4, (size_t)4 * 32 * (2 * D + 32));
     const bool inl = p.n_inline != 0;
 #define SV_ATTN3(DD, N, B)                                                          \
@@ -812,7 +847,7 @@ sv_status attn_params_fill(void* out, const sv_shape* sh, const float* qkv, cons
                            uint32_t n_runs, uint32_t max_run, const uint32_t* vis, float* o, float* part_o,
                            float* part_l) {
   if (!out || !sh || !kv || !args || !host_runs) return fail(SV_ERR_ARG, "layers: attention arguments");
-  if (n_runs == 0 || n_runs > SV_INLINE_RUNS) return fail(SV_ERR_UNSUPPORTED, "layers: %u attention runs", n_runs);
+  if (n_runs == 0 || n_runs > SV_LAYERS_RUNS) return fail(SV_ERR_UNSUPPORTED, "layers: %u attention runs", n_runs);
   if (sh->head_dim != 64 || !kv->is_global || args->split % 32 || args->split > 32u * 4 * 4)
     return fail(SV_ERR_UNSUPPORTED, "layers: head_dim %u, global %u, split %u", sh->head_dim, kv->is_global, args->split);
   if (args->rope && !rope_rows) return fail(SV_ERR_ARG, "layers: rope rows missing");

@@ -6,7 +6,9 @@
 
 namespace sv {
 
-constexpr uint32_t SV_INLINE_RUNS = 32;
+// Runs a launch carries: every step of 32 streams and a prompt chunk of 768 rows in runs of 12.
+constexpr uint32_t SV_INLINE_RUNS = 64;
+constexpr uint32_t SV_LAYERS_RUNS = 32;  // the persistent layer kernel's limit
 
 struct AttnParams {
   const float* qkv;

@@ -422,6 +422,22 @@ def test_attn_verify_head_dim_128(gpu, runs_T, p0s, split, tree, rope):
     _attn_verify_case(runs_T, p0s, split, tree, rope, sh=SH128)
 
 
+@pytest.mark.parametrize("runs_T", [[5], [8, 1], [9], [12, 1, 4], [13, 16, 2]])
+@pytest.mark.parametrize("D", [64, 128])
+def test_attn_shared_query_build(gpu, runs_T, D):
+    """Two to four column tiles, each built by one wave: full and partial last tiles (20 to 64
+    columns), runs shorter than the launch's tiles (waves whose tile lies past the run), with and
+    without cached keys, against the oracle."""
+    banner(f"attn shared queries D={D} runs={runs_T}")
+    sel = C.c_int.in_dll(L.lib(), "_ZN2sv12g_attn_allinE")
+    sel.value = 0
+    try:
+        _attn_verify_case(runs_T, [(257, 0, 90)[i] for i in range(len(runs_T))], 64, False, 1,
+                          **({"sh": SH128} if D == 128 else {}))
+    finally:
+        sel.value = -1
+
+
 # ------------------------------------------------------------------------------ sampler
 def sample_rows(n, temps, top_ps, seed=11, pos0=100):
     rows = []

@@ -179,6 +179,25 @@ def test_multi_stream_steps(gpu):
         assert np.array_equal(res.ids, ids_r), "greedy ids diverged (margins within tolerance)"
 
 
+@pytest.mark.parametrize("n", [33, 64, 65])
+def test_run_headers_in_the_launch(gpu, n):
+    """A step of n one- to three-row runs against the oracle engine: up to 64 runs' headers (first
+    token, rows, slot) travel with the attention launch, 65 are read from memory."""
+    banner(f"{n} runs")
+    shape = ModelShape(n_layers=1, vocab=2048, vocab_real=2048)
+    ctxs = [7 * i % 200 for i in range(n)]
+    model, gm, eng, ref, slots, rng = build_pair(shape, ctx=ctxs, n_seqs=n, seed=11, max_seq_len=256,
+                                                 max_head_rows=3 * n)
+    for s in slots:
+        t = int(rng.integers(0, shape.vocab_real))
+        eng.set_feed(s, ref.seq_len[s], t)
+        ref.set_feed(s, ref.seq_len[s], t)
+    runs = [(s, [L.FEED_ROW] + [int(x) for x in rng.integers(0, shape.vocab_real, i % 3)], True) for i, s in enumerate(slots)]
+    ids_r, logits_r, em_r, extra_r = ref.step(runs)
+    res = eng.step(runs, logits=True)
+    compare_step(res, ids_r, logits_r, em_r, extra_r, eng, ref, slots, runs=runs)
+
+
 def test_tree_step_compacts(gpu):
     """A 16-node draft tree whose accepted path is not a prefix: kv_compact must move the
     path's K/V to consecutive positions (compared bit for bit on the V cache)."""
