@@ -209,6 +209,11 @@ __device__ __forceinline__ void compute_batch_t(const AttnParams& p, const KvBat
                                                 const uint32_t (&clo)[NCT], const uint32_t* vis_cached = nullptr) {
   constexpr int KST = D / 32, VE = D / 16, NV = D / 32;
   const int c16 = lane & 15, q = lane >> 4;
+  // The product phases go at a raised wave priority where two waves of three or more column tiles
+  // share a SIMD (D = 64): the wave in its products keeps the matrix unit fed while the other does its
+  // exponentials, in place of both taking turns in the same phase (512 rows at 32768 keys: 261 -> 253
+  // us; at one wave per SIMD, D = 128, it measured slower: 68 -> 72).
+  constexpr bool PRIO = D == 64 && NCT >= 3;
   // V into the stage first (its LDS writes overlap the score products).
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
@@ -222,6 +227,7 @@ __device__ __forceinline__ void compute_batch_t(const AttnParams& p, const KvBat
       const uint32_t byte = 16 * lane + 1024 * v;
       *(u32x4*)((char*)stage + (16 * mt + byte / (2 * D)) * stage_row<D>() + byte % (2 * D)) = w;
     }
+  if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
   // S^T tiles: lane holds keys kb + 16 mt + 4 q + i, column 16 ct + c16.
   f32x4 S[2][NCT];
 #pragma unroll
@@ -237,6 +243,7 @@ __device__ __forceinline__ void compute_batch_t(const AttnParams& p, const KvBat
       }
       S[mt][ct] = a;
     }
+  if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
   bf16x8 ph[NCT], pl[NCT];
 #pragma unroll
   for (int ct = 0; ct < NCT; ct++) {
@@ -262,6 +269,7 @@ __device__ __forceinline__ void compute_batch_t(const AttnParams& p, const KvBat
       }
     split8(pv, ph[ct], pl[ct]);
   }
+  if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
   // O^T[dt] (rows: dims 16 dt + 4 q + i) += V^T[dt] P^T; the A operand's k slots 4 mt + t are
   // keys kb + 16 mt + 4 q + t (P's layout), read transposed: lane (i, q) addresses key
   // 4 q + i / 4 of tile mt, dims 16 dt + 4 (i % 4) .. + 3.
@@ -279,6 +287,7 @@ __device__ __forceinline__ void compute_batch_t(const AttnParams& p, const KvBat
       O[dt][ct] = mfma16(av, pl[ct], O[dt][ct]);
     }
   }
+  if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
 }
 
 // fp32 activation words at element offset `off` (a multiple of 4): plain, or coherent (sc1)
