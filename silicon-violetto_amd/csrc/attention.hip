@@ -4,7 +4,8 @@
 //
 // One workgroup (4 waves) per (key split s, kv head g, run r):
 //   - Columns are the run's T tokens x G query heads of kv head g (column c: token c / G,
-//     head g G + c % G), in NCT tiles of 16. Each lane builds its columns' queries in
+//     head g G + c % G), in NCT tiles of 16. Each lane builds its columns' queries (or, with
+//     attn_share_queries, one tile's, exchanged through LDS) in
 //     registers: rms-norm over the head (no gain), RoPE on pairs (2j, 2j+1), j < 32, times
 //     softmax scale * log2 e, split into bf16 hi + lo MFMA operands.
 //   - Splits own `split` cached keys each. The run's new keys (norm, RoPE, K and V rounded to

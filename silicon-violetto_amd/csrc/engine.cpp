@@ -203,7 +203,9 @@ constexpr uint32_t MAX_SPLIT = 3968 / 128 * 128;
 // workgroups per compute unit (rounded up):
 //   one workgroup per compute unit: its dependent-load chain, 9.7 + 1.2 b;
 //   more: they share the unit's throughput, k (F + 1.05 b), F = 5.3 (<= 32 columns per kv
-//   head) or 19 (more: 4x the query, reduction and partial traffic per workgroup).
+//   head) or 19 (more: 4x the query, reduction and partial traffic per workgroup; the kernel's own fixed
+//   part is about 8 by now, but 8 and 13 chose splits no faster: 512 rows at 32768 keys 270 and 263 us,
+//   266 with 19).
 // The larger of the two; ties go to the smaller split. Contexts are counted at the plan's
 // furthest replay (cached + extra keys).
 uint32_t choose_split(const std::vector<uint32_t>& cached, uint32_t extra, uint32_t nkv, uint32_t max_run,
