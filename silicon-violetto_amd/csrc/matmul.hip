@@ -1187,6 +1187,13 @@ struct GemmCfg {
   uint32_t bn() const { return tw() * nt; }
   uint32_t acc_bytes() const { return (uint32_t)(rtw * nt) * tw() * tw() / 16; }  // per thread
 };
+// The partial sums of a launch whose k is split (the sums of squares are fewer). The kernels address
+// them by a 32-bit offset through a descriptor of 2 GiB: a launch with more of them drops stores.
+static size_t gemm_part_bytes(uint32_t n, uint32_t m, const GemmCfg& c) {
+  return c.s <= 1 ? 0 : (size_t)(m / c.bm()) * ((n + c.bn() - 1) / c.bn()) * c.s * 64 * c.nw * c.acc_bytes();
+}
+constexpr size_t PART_LIMIT = (size_t)1 << 31;
+
 GemmTune g_gemm_tune;  // all zero: the built-in choice
 int g_gemm_order = -1;  // tests: force a work order (-1: the modelled choice)
 
@@ -1215,6 +1222,7 @@ static GemmCfg pick_tiles32(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
     const uint64_t cells = (uint64_t)(m / bm) * ((n + bn - 1) / bn);
     for (uint32_t s : {1u, 2u, 4u, 8u}) {
       if (nch % s || (s > 1 && nch / s < 4)) continue;
+      if (gemm_part_bytes(n, m, GemmCfg{sh.rt, sh.nt, (int)s, 4, sh.mf, 8, sh.cpi}) >= PART_LIMIT) continue;
       const uint64_t wgs = cells * s;
       float us = (float)((wgs + 255) / 256) * (3.5f + (nch / s) * sh.us);
       if (s > 1) us += std::min(1.0f, wgs / 256.0f) * (2.5f + 0.8f * s) * sh.merge;
@@ -1228,11 +1236,7 @@ static GemmCfg pick_tiles32(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
 // 17-512 rows: 32-token blocks (NT = 2) of two row tiles per wave with two k splits, four when that
 // leaves fewer than 256 workgroups; one row tile per wave when the splits alone cannot reach 256
 // workgroups, and with int8 scale groups shorter than k.
-static GemmCfg pick_gemm(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
-  if (g_gemm_tune.rtw)
-    return GemmCfg{g_gemm_tune.rtw, g_gemm_tune.nt, std::max(1, g_gemm_tune.s), g_gemm_tune.d ? g_gemm_tune.d : 4,
-                   g_gemm_tune.mf ? g_gemm_tune.mf : 16, g_gemm_tune.nw ? g_gemm_tune.nw : 4,
-                   g_gemm_tune.cpi ? g_gemm_tune.cpi : 1};
+static GemmCfg pick_builtin(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   const uint32_t nch = k / GKC;
   const uint64_t tiles = (uint64_t)(m / 256) * ((n + 31) / 32) * nch;  // 256-row x 32-token x 64-k blocks
   const bool big = (uint64_t)m * k * (fmt == SV_FMT_I8 ? 1 : 2) > (96ull << 20);
@@ -1303,6 +1307,18 @@ static GemmCfg pick_gemm(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uin
   return c;
 }
 
+// The launch of a GEMM: the tests' override or the built-in choice, whose k splits (powers of two)
+// are halved until the partial sums fit their descriptor.
+static GemmCfg pick_gemm(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
+  if (g_gemm_tune.rtw)
+    return GemmCfg{g_gemm_tune.rtw, g_gemm_tune.nt, std::max(1, g_gemm_tune.s), g_gemm_tune.d ? g_gemm_tune.d : 4,
+                   g_gemm_tune.mf ? g_gemm_tune.mf : 16, g_gemm_tune.nw ? g_gemm_tune.nw : 4,
+                   g_gemm_tune.cpi ? g_gemm_tune.cpi : 1};
+  GemmCfg c = pick_builtin(fmt, grouped, n, m, k);
+  while (gemm_part_bytes(n, m, c) >= PART_LIMIT) c.s /= 2;
+  return c;
+}
+
 static size_t gemm_ws_layout(uint32_t n, uint32_t m, const GemmCfg& c, size_t* ss_off, size_t* part_off) {
   if (c.s <= 1) return 0;
   const size_t n_tblk = (n + c.bn() - 1) / c.bn(), cells = m / c.bm() * n_tblk;
@@ -1310,7 +1326,7 @@ static size_t gemm_ws_layout(uint32_t n, uint32_t m, const GemmCfg& c, size_t* s
   *ss_off = off;
   off += (cells * c.s * c.bn() * 4 + 255) / 256 * 256;
   *part_off = off;
-  off += cells * c.s * 64 * c.nw * c.acc_bytes();
+  off += gemm_part_bytes(n, m, c);
   return off;
 }
 
@@ -1435,6 +1451,8 @@ static sv_status gemm_launch(hipStream_t stream, uint32_t fmt, MMParams& p, void
   size_t ss_off = 0, part_off = 0;
   const size_t need = gemm_ws_layout(p.n, p.m, c, &ss_off, &part_off);
   if (need) {
+    if (gemm_part_bytes(p.n, p.m, c) >= PART_LIMIT)
+      return fail(SV_ERR_UNSUPPORTED, "matmul (gemm): %d k splits of 2 GiB or more of partial sums", c.s);
     if ((size_t)rb * n_tblk > COUNTER_SLOTS) return fail(SV_ERR_UNSUPPORTED, "matmul (gemm): cells exceed the counters");
     if (!ws || ws_bytes < need)
       return fail(SV_ERR_ARG, "matmul: workspace %zu < %zu bytes (sv_matmul_workspace_bytes)", ws_bytes, need);

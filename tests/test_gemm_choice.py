@@ -1,0 +1,53 @@
+"""The GEMM's launch choice as a caller sees it without a GPU: the workspace its k splits ask for,
+and the launches it refuses."""
+from __future__ import annotations
+
+import ctypes as C
+
+import pytest
+import torch
+
+from violetto import _lib as L
+
+COUNTERS = 65536 * 4           # hand-off counters at the front of a workspace
+WINDOW = 1 << 31               # bytes of partial sums the kernels can address
+
+
+def partials_at_most(nbytes: int) -> int:
+    """Bytes of partial sums in a workspace (the rest: the counters and a sum of squares per
+    token and split, at most 1/64 of the partials)."""
+    return max(0, nbytes - COUNTERS)
+
+
+@pytest.mark.parametrize("m,k", [(28672, 8192), (28672, 4096), (151552, 4096), (27648, 5120), (16384, 8192),
+                                 (2048, 8192), (16384, 2048), (32000, 2048), (1280, 3328), (6656, 1280),
+                                 (8256, 8192), (40000, 8192)])
+def test_split_partials_stay_addressable(m, k):
+    """Partial sums are addressed by 32-bit offsets through a 2 GiB descriptor: no row count asks
+    for more of them (past it stores were dropped and the sums read back as zeros)."""
+    rows = sorted({int(17 * 1.07 ** i) for i in range(115)} | {513, 1025, 1682, 4609, 4770, 8200, 9345, 16385, 63361})
+    for n in rows:
+        if n * k * 4 >= WINDOW:
+            continue
+        got = L.lib().sv_matmul_workspace_bytes(n, m, k)
+        assert partials_at_most(got) < WINDOW + WINDOW // 64, f"{n} rows: workspace of {got} bytes"
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up pointers: the call must not reach a GPU")
+def test_launch_past_the_window_is_refused():
+    """A forced split (the tests' override) with 2 GiB of partial sums or more is refused before
+    any launch; the same shape one step below is not (without a device it fails at the launch)."""
+    tune = (C.c_int * 7).in_dll(L.lib(), "_ZN2sv11g_gemm_tuneE")
+    m, k = 16384, 2048
+    one = C.c_void_p(1 << 20)
+    try:
+        for i, v in enumerate((1, 1, 4, 4, 33, 8, 2)):
+            tune[i] = v
+        for n, ok in ((8192, False), (8192 - 32, True)):   # m x n x 4 splits x 4 bytes
+            mat = L.Matrix(one, one, m, k, L.FMT_I8, 31)
+            a = L.MatArgs(n, k, m, L.EPI_RAW, 0, m, 1.0, 0, 0, 1, k, 31)
+            rc = L.lib().sv_matmul(None, C.byref(mat), one, None, one, None, None, C.byref(a), one, 1 << 40)
+            assert (rc == 4) == (not ok), L.lib().sv_last_error()
+    finally:
+        for i in range(7):
+            tune[i] = 0
