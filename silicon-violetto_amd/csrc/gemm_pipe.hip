@@ -3,7 +3,7 @@
 
 namespace sv {
 
-// The GEMM for the rows that fill 32 x 32 tiles (matmul.hip pick_tiles32): 8 waves, BM = 256 RT
+// The GEMM for the rows that fill 32 x 32 tiles (matmul.hip pick_by_time): 8 waves, BM = 256 RT
 // output rows (RT 32-row tiles per wave), BN = 32 NT tokens, 1/S of k; iterations of CPI chunks of
 // 64 k. Operands and layouts are mm_gemm32's (weights straight to registers in MFMA lane order
 // and converted there, X split once per workgroup to bf16 hi + lo in LDS). What differs:

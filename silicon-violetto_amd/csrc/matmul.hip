@@ -1197,64 +1197,72 @@ constexpr size_t PART_LIMIT = (size_t)1 << 31;
 GemmTune g_gemm_tune;  // all zero: the built-in choice
 int g_gemm_order = -1;  // tests: force a work order (-1: the modelled choice)
 
-// The 32 x 32-tile launch with the least modelled time (us, fitted on MI355X at 96-2048 rows with
-// the weights cold): rounds of 256 workgroups (one per compute unit), each 3.5 for its first loads
-// and its stores plus its 64-k chunks at the shape's time per chunk with the chip busy (mm_gemm32's
-// 256 x 32 block 0.55; mm_pipe's 256 x 32 0.60, 256 x 64 1.04, 512 x 32 1.10, 256 x 128 1.85,
-// 512 x 64 1.74, 512 x 128 3.2: the larger the block, the fewer operand bytes and conversions per
-// product); a split of k adds its partial sums, written and read back by the last split. The
-// blocks of 512 rows hold two sets of sums with scale groups, and spill: not offered there.
-static GemmCfg pick_tiles32(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
+// The launch with the least modelled time (us), for work that fills 256-row blocks. A launch runs in
+// rounds of the blocks that the device holds at once (256 of mm_pipe and mm_gemm32, one per compute
+// unit; 512 of mm_gemm's blocks of four waves). A round takes 7.6 for its first loads, its stores and
+// its slowest block, plus the block's 64-k chunks at a time per chunk between lo (few compute units
+// busy: a higher clock, more of the memory each) and hi (all of them). A split of k pays for its
+// partial sums, and only splits within one round are offered: in several rounds the sums of every
+// round are written and read back at 0.5-1 us a MB, where a round saved is worth less (gate_up,
+// 16384 x 2048, at 1152 rows: 330 us in four splits of five rounds, 336 MB, 159 unsplit; down, 2048 x
+// 8192, at 1500 rows 188 in eight splits, 102 in two). The blocks of 512 rows hold two sets of sums
+// with scale groups, and spill: not offered there; mm_gemm's (no conversions to hide) with bf16 only.
+// Fitted on MI355X to 1900 launches at 40-2048 rows of the 2048- and 1280-wide models' matrices,
+// weights cold: over 247 (matrix, format, rows) the choice is 0.1 % slower than the fastest launch
+// measured on average, 5 % at most.
+static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   static const struct {
-    int rt, nt, cpi, mf;
-    float us, merge;  // per chunk; of the partial sums' cost, (rt nt)^0.6
-  } SHAPES[] = {{1, 1, 1, 32, 0.55f, 1.0f}, {1, 1, 2, 33, 0.60f, 1.0f}, {1, 2, 2, 33, 1.04f, 1.5f},
-                {2, 1, 1, 33, 1.10f, 1.5f}, {1, 4, 1, 33, 1.85f, 2.3f}, {2, 2, 1, 33, 1.74f, 2.3f},
-                {2, 4, 1, 33, 3.2f, 3.5f}};
+    GemmCfg c;
+    float lo, hi, merge;  // us per chunk; of a split's cost, (row tiles x token tiles)^0.9
+  } SHAPES[] = {{{1, 1, 1, 4, 32, 8, 1}, 0.39f, 0.49f, 1.0f},  {{1, 1, 1, 4, 33, 8, 2}, 0.41f, 0.58f, 1.0f},
+                {{1, 2, 1, 4, 33, 8, 2}, 0.63f, 0.92f, 1.87f}, {{2, 1, 1, 4, 33, 8, 1}, 0.86f, 1.00f, 1.87f},
+                {{1, 4, 1, 4, 33, 8, 1}, 1.13f, 1.83f, 3.48f}, {{2, 2, 1, 4, 33, 8, 1}, 1.09f, 1.62f, 3.48f},
+                {{2, 4, 1, 4, 33, 8, 1}, 2.06f, 3.22f, 6.50f}, {{4, 4, 1, 2, 16, 4, 1}, 1.04f, 1.91f, 0.0f},
+                {{2, 5, 1, 2, 16, 4, 1}, 1.15f, 1.37f, 0.0f}};
   const uint32_t nch = k / GKC;
+  const float pipe = grouped ? 1.23f : fmt == SV_FMT_BF16 ? 1.03f : 1.0f;  // mm_pipe's chunks by format
   GemmCfg best{1, 1, 1, 4, 33, 8, 2};
   float best_us = 1e30f;
   for (const auto& sh : SHAPES) {
-    if (sh.mf == 32 && (grouped || fmt != SV_FMT_I8)) continue;
-    if (grouped && sh.rt == 2 && sh.nt > 1) continue;
-    const uint32_t bm = 256u * sh.rt, bn = 32u * sh.nt;
-    if (m % bm) continue;
-    const uint64_t cells = (uint64_t)(m / bm) * ((n + bn - 1) / bn);
-    for (uint32_t s : {1u, 2u, 4u, 8u}) {
-      if (nch % s || (s > 1 && nch / s < 4)) continue;
-      if (gemm_part_bytes(n, m, GemmCfg{sh.rt, sh.nt, (int)s, 4, sh.mf, 8, sh.cpi}) >= PART_LIMIT) continue;
-      const uint64_t wgs = cells * s;
-      float us = (float)((wgs + 255) / 256) * (3.5f + (nch / s) * sh.us);
-      if (s > 1) us += std::min(1.0f, wgs / 256.0f) * (2.5f + 0.8f * s) * sh.merge;
-      if (us < best_us) best_us = us, best = GemmCfg{sh.rt, sh.nt, (int)s, 4, sh.mf, 8, sh.cpi};
+    GemmCfg c = sh.c;
+    if (c.mf == 32 && (grouped || fmt != SV_FMT_I8)) continue;
+    if (c.mf == 16 && fmt != SV_FMT_BF16) continue;
+    if (grouped && c.rtw == 2 && c.nt > 1) continue;
+    if (m % c.bm()) continue;
+    const uint64_t cells = (uint64_t)(m / c.bm()) * ((n + c.bn() - 1) / c.bn()), slots = c.mf == 16 ? 512 : 256;
+    for (int s : {1, 2, 4, 8}) {
+      if (s > 1 && (c.mf == 16 || nch % s || nch / s < 4 || cells * s > slots)) continue;
+      const uint64_t rounds = (cells * s + slots - 1) / slots;
+      const float fill = (float)(cells * s) / (float)(rounds * slots);
+      float us = rounds * (7.57f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
+      if (s > 1) us += fill * (2.7f + 0.67f * s) * sh.merge;
+      if (us < best_us) {
+        c.s = s;
+        best_us = us, best = c;
+      }
     }
   }
   return best;
 }
 
-// Built-in choice below the 32 x 32 tiles' range (pick_tiles32), from measurements on MI355X at
-// 17-512 rows: 32-token blocks (NT = 2) of two row tiles per wave with two k splits, four when that
-// leaves fewer than 256 workgroups; one row tile per wave when the splits alone cannot reach 256
-// workgroups, and with int8 scale groups shorter than k.
+// Built-in choice: pick_by_time where the work fills its blocks; below that, from measurements on
+// MI355X at 17-512 rows, 32-token blocks (NT = 2) of two row tiles per wave with two k splits, four
+// when that leaves fewer than 256 workgroups; one row tile per wave when the splits alone cannot
+// reach 256 workgroups, and with int8 scale groups shorter than k.
 static GemmCfg pick_builtin(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   const uint32_t nch = k / GKC;
   const uint64_t tiles = (uint64_t)(m / 256) * ((n + 31) / 32) * nch;  // 256-row x 32-token x 64-k blocks
   const bool big = (uint64_t)m * k * (fmt == SV_FMT_I8 ? 1 : 2) > (96ull << 20);
-  // The 32 x 32 tiles, wherever the work fills them (m a multiple of 256). Both sides measured on
-  // MI355X at 24-2048 rows, weights cold:
-  //  - int8 with a scale per row: from 96 rows (gate_up 96 rows 27.5 -> 23.1 us, 2048 rows 290 ->
-  //    213; below, the 16-wide tiles: qkv 64 rows 12.1 against 12.8);
+  // pick_by_time (m a multiple of 256). Both sides measured on MI355X at 17-2048 rows, weights cold:
+  //  - int8 with a scale per row: from 96 rows (gate_up 96 rows 27.5 -> 23.1 us; below, the 16-wide
+  //    tiles: qkv 64 rows 12.1 against 12.8);
   //  - int8 in scale groups: from 1500 blocks (gate_up of the 1280-wide model at 512 rows 47 -> 27,
-  //    at 2048 187 -> 87, down at 256 27 -> 21; below, o at 256 rows 14.5 against 15.7);
-  //  - bf16: from 4096 blocks (gate_up 192 rows 54 -> 38, 2048 rows 337 -> 265; below, o at 256
-  //    rows 16.2 against 17.4);
-  //  - bf16 weights too large to stay cached (the 131 MB head): from 49 rows (64 rows 46 -> 39,
-  //    256 rows 113 -> 75), but two 80-token blocks at 129-160 rows (63 against 66).
+  //    down at 256 27 -> 21; below, o at 256 rows 14.5 against 15.7);
+  //  - bf16: above 4096 blocks (gate_up 192 rows 54 -> 38; at 4096, o at 512 rows 19.2 against 20.2);
+  //  - bf16 weights too large to stay cached (the 131 MB head): from 49 rows (64 rows 46 -> 39).
   if (m % 256 == 0) {
-    const bool wide = fmt == SV_FMT_I8 ? (grouped ? tiles >= 1500 : n >= 96)
-                      : big            ? n > 48 && (n <= 128 || n > 160)
-                                       : tiles >= 4096;
-    if (wide) return pick_tiles32(fmt, grouped, n, m, k);
+    const bool wide = fmt == SV_FMT_I8 ? (grouped ? tiles >= 1500 : n >= 96) : big ? n > 48 : tiles > 4096;
+    if (wide) return pick_by_time(fmt, grouped, n, m, k);
   }
   // Weights too large to stay cached between token blocks (the 131 MB bf16 head) are re-read
   // from HBM by every token block: below that shape, the fewest token blocks (48 or 80 tokens,

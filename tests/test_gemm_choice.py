@@ -33,6 +33,16 @@ def test_split_partials_stay_addressable(m, k):
         assert partials_at_most(got) < WINDOW + WINDOW // 64, f"{n} rows: workspace of {got} bytes"
 
 
+@pytest.mark.parametrize("m,k", [(3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (32000, 2048), (1792, 1280),
+                                 (1280, 1280), (6656, 1280), (1280, 3328)])
+def test_splits_stay_within_one_round(m, k):
+    """A split launch is at most one round of 256 workgroups of 512 x 128 sums (64 MiB) at any
+    row count: in several rounds the partial sums cost more than the rounds they save."""
+    for n in range(17, 2600):
+        got = partials_at_most(L.lib().sv_matmul_workspace_bytes(n, m, k))
+        assert got <= (64 << 20) * 65 // 64, f"{n} rows: workspace of {got} bytes"
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="made-up pointers: the call must not reach a GPU")
 def test_launch_past_the_window_is_refused():
     """A forced split (the tests' override) with 2 GiB of partial sums or more is refused before

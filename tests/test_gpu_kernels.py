@@ -741,6 +741,40 @@ def test_matmul_head_many_cells(gpu):
     close(got, ref, atol=5e-5 * 23, rtol=1e-4, what="head at 256 rows")
 
 
+@pytest.mark.parametrize("fmt,m,k,n", [("i8", 16384, 2048, 576), ("i8", 16384, 2048, 1152), ("bf16", 16384, 2048, 1100),
+                                       ("i8", 2048, 8192, 128), ("i8", 2048, 8192, 1409), ("bf16", 2048, 8192, 768),
+                                       ("i8", 3072, 2048, 704), ("bf16", 32000, 2048, 150), ("bf16", 32000, 2048, 300),
+                                       ("bf16", 32000, 2048, 577), ("g64", 6656, 1280, 600), ("g64", 1280, 3328, 1500)])
+def test_matmul_built_in_choice(gpu, fmt, m, k, n):
+    """The built-in launch at row counts between and past the blocks' sizes (one and several rounds of
+    blocks, k splits, the 16-wide blocks of 64 and 80 tokens with bf16), with the workspace that the
+    query asks for: EPI_NORM with the inverse norms of every row, a seeded sample of rows against the
+    oracle (sums of k products: 5e-5 of the largest value, as for the shapes above)."""
+    banner(f"built-in choice {fmt} m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + n)
+    w = torch.from_numpy(rng.normal(0, 0.02, (m, k)).astype(np.float32))
+    if fmt == "bf16":
+        host, sc, gs = bf16_bits(w.numpy()), None, 0
+        mat = K.matrix(u16_dev_bf16(host)).tiled()
+    else:
+        q, s = quantize_rows(w) if fmt == "i8" else quantize_groups(w, 64)
+        host, sc, gs = q.numpy(), s.view(torch.int16).numpy().view(np.uint16), 31 if fmt == "i8" else 6
+        mat = K.matrix(q.cuda(), s.cuda(), gs).tiled()
+    x = (rng.normal(0, 1, (n, k)) * rng.uniform(0.5, 4, (n, 1))).astype(np.float32)
+    rows = np.sort(np.append(rng.choice(n - 1, 5, replace=False), n - 1)).astype(np.uint32)
+    a = L.MatArgs(len(rows), k, m, L.EPI_NORM, 0, m, 0.75, 0.0, 0.0, 1, k, gs)
+    ref = oracle.matmul(L, host, sc, gs, x, a, x_rows=rows)
+    ws = K.Workspace(L.lib().sv_matmul_workspace_bytes(n, m, k))
+    for call in range(2):
+        y = torch.zeros(n, m, device="cuda")
+        aux = torch.zeros(n, device="cuda")
+        K.matmul(mat, to_dev(x), y, n=n, epi=L.EPI_NORM, flags=L.FLAG_WRITE_INV, scale=0.75, aux=aux, ws=ws)
+        torch.cuda.synchronize()
+        close(y.cpu().numpy()[rows], ref, atol=5e-5 * max(float(np.abs(ref).max()), 1.0), rtol=1e-4, what=f"call {call}")
+        inv = 1.0 / np.sqrt((x.astype(np.float64) ** 2).mean(1) + 2.0 ** -23)
+        close(aux.cpu().numpy(), inv.astype(np.float32), atol=1e-5, rtol=1e-4, what="inverse norms")
+
+
 @pytest.mark.parametrize("shape", [(1, 2, 1, 4), (2, 2, 2, 4), (2, 2, 4, 8), (1, 3, 2, 8), (2, 3, 1, 4),
                                                   (2, 4, 2, 4), (1, 5, 4, 4), (2, 5, 1, 4), (2, 8, 2, 4), (1, 8, 1, 4),
                                                   (4, 4, 1, 4), (4, 2, 2, 4), (4, 5, 4, 4), (4, 4, 2, 2), (4, 3, 1, 2),
