@@ -1197,49 +1197,73 @@ constexpr size_t PART_LIMIT = (size_t)1 << 31;
 GemmTune g_gemm_tune;  // all zero: the built-in choice
 int g_gemm_order = -1;  // tests: force a work order (-1: the modelled choice)
 
-// The launch with the least modelled time (us), for work that fills 256-row blocks. A launch runs in
-// rounds of the blocks that the device holds at once (256 of mm_pipe and mm_gemm32, one per compute
-// unit; 512 of mm_gemm's blocks of four waves). A round takes 7.6 for its first loads, its stores and
-// its slowest block, plus the block's 64-k chunks at a time per chunk between lo (few compute units
-// busy: a higher clock, more of the memory each) and hi (all of them). A split of k pays for its
-// partial sums, and only splits within one round are offered: in several rounds the sums of every
-// round are written and read back at 0.5-1 us a MB, where a round saved is worth less (gate_up,
-// 16384 x 2048, at 1152 rows: 330 us in four splits of five rounds, 336 MB, 159 unsplit; down, 2048 x
-// 8192, at 1500 rows 188 in eight splits, 102 in two). The blocks of 512 rows hold two sets of sums
-// with scale groups, and spill: not offered there; mm_gemm's (no conversions to hide) with bf16 only.
-// Fitted on MI355X to 1900 launches at 40-2048 rows of the 2048- and 1280-wide models' matrices,
-// weights cold: over 247 (matrix, format, rows) the choice is 0.1 % slower than the fastest launch
-// measured on average, 5 % at most.
+// The launch with the least modelled time (us), for work that fills 256-row blocks.
+//  - mm_pipe and mm_gemm32 run in rounds of 256 blocks, one per compute unit. A round takes 5.9 for its
+//    first loads, its stores and its slowest block, plus the block's 64-k chunks at a time per chunk
+//    between lo (few compute units busy: a higher clock, more of the memory each) and hi (all of them).
+//    A split of k pays for its partial sums, and only splits within one round are offered: in several
+//    rounds the sums of every round are written and read back at 0.5-1 us a MB, where a round saved is
+//    worth less (gate_up, 16384 x 2048, at 1152 rows: 330 us in four splits of five rounds, 336 MB, 159
+//    unsplit; down, 2048 x 8192, at 1500 rows 188 in eight splits, 102 in two). The blocks of 512 rows
+//    hold two sets of sums with scale groups, and spill: not offered there.
+//  - mm_gemm's blocks of 64 and 80 tokens (bf16 only: there are no conversions to hide) run two a compute
+//    unit, 512 a round: lo up to 256 of them, hi as soon as some unit has two (the bf16 head, 32000 x
+//    2048, at 192 rows: 375 blocks of 64 tokens 79 us, mm_pipe's 250 blocks of 128 tokens 68).
+//  - mm_gemm's splits of 32-token blocks (128 rows in two with bf16, 64 rows in two to eight with scale
+//    groups): a time linear in blocks and chunks while one round holds them all, three blocks a compute
+//    unit, four with groups (bf16 qkv, 3072 x 2048: 768 blocks at 512 rows 26 us, 816 at 513 rows 28).
+//    They win where the 32-wide blocks are few (qkv at 352 rows 22 us against 25; gate_up in groups at 32
+//    rows 20 against 24).
+// Fitted on MI355X to 7400 launches at 17-2048 rows of the 2048- and 1280-wide models' matrices and
+// heads with their own epilogues, weights cold: over 674 (matrix, format, rows) the choice is 2.0 %
+// slower on average than the fastest of all launches measured, and 4 % at most slower than the better
+// one of the two rules that it replaced (at 6 points more than 3 %).
 static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   static const struct {
     GemmCfg c;
-    float lo, hi, merge;  // us per chunk; of a split's cost, (row tiles x token tiles)^0.9
-  } SHAPES[] = {{{1, 1, 1, 4, 32, 8, 1}, 0.39f, 0.49f, 1.0f},  {{1, 1, 1, 4, 33, 8, 2}, 0.41f, 0.58f, 1.0f},
-                {{1, 2, 1, 4, 33, 8, 2}, 0.63f, 0.92f, 1.87f}, {{2, 1, 1, 4, 33, 8, 1}, 0.86f, 1.00f, 1.87f},
-                {{1, 4, 1, 4, 33, 8, 1}, 1.13f, 1.83f, 3.48f}, {{2, 2, 1, 4, 33, 8, 1}, 1.09f, 1.62f, 3.48f},
-                {{2, 4, 1, 4, 33, 8, 1}, 2.06f, 3.22f, 6.50f}, {{4, 4, 1, 2, 16, 4, 1}, 1.04f, 1.91f, 0.0f},
-                {{2, 5, 1, 2, 16, 4, 1}, 1.15f, 1.37f, 0.0f}};
+    float lo, hi;  // us per chunk
+  } SHAPES[] = {{{1, 1, 1, 4, 32, 8, 1}, 0.44f, 0.55f}, {{1, 1, 1, 4, 33, 8, 2}, 0.49f, 0.67f},
+                {{1, 2, 1, 4, 33, 8, 2}, 0.77f, 0.95f}, {{2, 1, 1, 4, 33, 8, 1}, 0.98f, 1.07f},
+                {{1, 4, 1, 4, 33, 8, 1}, 1.33f, 1.56f}, {{2, 2, 1, 4, 33, 8, 1}, 1.32f, 1.54f},
+                {{2, 4, 1, 4, 33, 8, 1}, 2.23f, 3.03f}, {{4, 4, 1, 2, 16, 4, 1}, 1.28f, 1.77f},
+                {{2, 5, 1, 2, 16, 4, 1}, 1.12f, 1.41f}};
   const uint32_t nch = k / GKC;
-  const float pipe = grouped ? 1.23f : fmt == SV_FMT_BF16 ? 1.03f : 1.0f;  // mm_pipe's chunks by format
+  const float pipe = grouped ? 1.28f : fmt == SV_FMT_BF16 ? 1.06f : 1.0f;  // mm_pipe's chunks by format
   GemmCfg best{1, 1, 1, 4, 33, 8, 2};
   float best_us = 1e30f;
+  auto offer = [&](GemmCfg c, int s, float us) {
+    if (us < best_us) c.s = s, best_us = us, best = c;
+  };
+  auto cells_of = [&](const GemmCfg& c) { return (uint64_t)(m / c.bm()) * ((n + c.bn() - 1) / c.bn()); };
   for (const auto& sh : SHAPES) {
-    GemmCfg c = sh.c;
-    if (c.mf == 32 && (grouped || fmt != SV_FMT_I8)) continue;
-    if (c.mf == 16 && fmt != SV_FMT_BF16) continue;
-    if (grouped && c.rtw == 2 && c.nt > 1) continue;
+    const GemmCfg& c = sh.c;
     if (m % c.bm()) continue;
-    const uint64_t cells = (uint64_t)(m / c.bm()) * ((n + c.bn() - 1) / c.bn()), slots = c.mf == 16 ? 512 : 256;
+    const uint64_t cells = cells_of(c);
+    if (c.mf == 16) {
+      if (fmt != SV_FMT_BF16) continue;
+      const uint64_t rem = cells % 512;
+      float us = cells / 512 * (3.55f + nch * sh.hi);
+      if (rem) us += 3.55f + nch * (rem <= 256 ? sh.lo : sh.hi);
+      offer(c, 1, us);
+      continue;
+    }
+    if (c.mf == 32 && (grouped || fmt != SV_FMT_I8)) continue;
+    if (grouped && c.rtw == 2 && c.nt > 1) continue;
     for (int s : {1, 2, 4, 8}) {
-      if (s > 1 && (c.mf == 16 || nch % s || nch / s < 4 || cells * s > slots)) continue;
-      const uint64_t rounds = (cells * s + slots - 1) / slots;
-      const float fill = (float)(cells * s) / (float)(rounds * slots);
-      float us = rounds * (7.57f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
-      if (s > 1) us += fill * (2.7f + 0.67f * s) * sh.merge;
-      if (us < best_us) {
-        c.s = s;
-        best_us = us, best = c;
-      }
+      if (s > 1 && (nch % s || nch / s < 4 || cells * s > 256)) continue;
+      const uint64_t rounds = (cells * s + 255) / 256;
+      const float fill = (float)(cells * s) / (float)(rounds * 256);
+      float us = rounds * (5.93f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
+      if (s > 1) us += fill * (c.mf == 32 ? 5.32f + 0.51f * s : (2.51f + 0.98f * s) * (c.rtw * c.nt));
+      offer(c, s, us);
+    }
+  }
+  if (grouped || fmt == SV_FMT_BF16) {
+    const GemmCfg c{grouped ? 1 : 2, 2, 1, 2};
+    for (int s : {2, 4, 8}) {
+      if ((s > 2 && !grouped) || nch % s || nch / s < 4 || cells_of(c) * s > (grouped ? 1024u : 768u)) continue;
+      const float x = cells_of(c) * s / 512.0f, ch = (float)(nch / s);
+      offer(c, s, grouped ? 0.04f + 0.82f * ch + x * (2.28f + 0.40f * ch) : -0.20f + 0.60f * ch + x * (4.82f + 0.36f * ch));
     }
   }
   return best;
@@ -1325,6 +1349,13 @@ static GemmCfg pick_gemm(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uin
   GemmCfg c = pick_builtin(fmt, grouped, n, m, k);
   while (gemm_part_bytes(n, m, c) >= PART_LIMIT) c.s /= 2;
   return c;
+}
+
+// The launch of a GEMM as numbers (tests: the choice is checked against measured times without a GPU).
+void gemm_choice(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k, int out[7]) {
+  const GemmCfg c = pick_gemm(fmt, grouped, n, m, k);
+  const int v[7] = {c.rtw, c.nt, c.s, c.d, c.mf, c.nw, c.cpi};
+  std::copy(v, v + 7, out);
 }
 
 static size_t gemm_ws_layout(uint32_t n, uint32_t m, const GemmCfg& c, size_t* ss_off, size_t* part_off) {

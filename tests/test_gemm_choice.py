@@ -61,3 +61,31 @@ def test_launch_past_the_window_is_refused():
     finally:
         for i in range(7):
             tune[i] = 0
+
+
+# (format, m, k, rows) -> measured us of launches (row tiles per wave, token tiles, k splits, chunks in
+# flight, tile: 16 mm_gemm, 32 mm_gemm32, 33 mm_pipe, waves, chunks per iteration), MI355X, weights cold:
+# sizes at which a rule of this choice has taken a launch 5-40 % slower than another one.
+MEASURED = [
+    ("bf16", 32000, 2048, 161, {(1, 4, 1, 4, 33, 8, 1): 64.8, (4, 4, 1, 2, 16, 4, 1): 77.4, (2, 3, 1, 4, 16, 4, 1): 79.4}),
+    ("bf16", 32000, 2048, 192, {(1, 4, 1, 4, 33, 8, 1): 67.6, (4, 4, 1, 2, 16, 4, 1): 79.4, (2, 3, 1, 4, 16, 4, 1): 81.6}),
+    ("bf16", 32000, 2048, 448, {(1, 4, 1, 4, 33, 8, 1): 132.6, (4, 4, 1, 2, 16, 4, 1): 148.5}),
+    ("bf16", 3072, 2048, 352, {(2, 2, 2, 2, 16, 4, 1): 22.3, (1, 1, 1, 4, 33, 8, 2): 25.5}),
+    ("bf16", 3072, 2048, 384, {(2, 2, 2, 2, 16, 4, 1): 22.6, (1, 1, 1, 4, 33, 8, 2): 25.3}),
+    ("bf16", 1280, 3328, 832, {(2, 2, 2, 2, 16, 4, 1): 28.7, (1, 2, 2, 4, 33, 8, 2): 32.2}),
+    ("bf16", 16384, 2048, 1280, {(4, 4, 1, 2, 16, 4, 1): 173.5, (2, 2, 1, 4, 33, 8, 1): 176.3}),
+    ("i8", 16384, 2048, 1152, {(2, 2, 1, 4, 33, 8, 1): 159.5, (2, 4, 4, 4, 33, 8, 1): 330.0}),
+    ("i8", 2048, 8192, 896, {(1, 2, 2, 4, 33, 8, 2): 70.6, (2, 2, 4, 4, 33, 8, 1): 75.6, (1, 1, 1, 4, 32, 8, 1): 79.7}),
+    ("i8", 2048, 8192, 1536, {(2, 2, 2, 4, 33, 8, 1): 106.5, (1, 1, 1, 4, 32, 8, 1): 143.4, (2, 2, 8, 4, 33, 8, 1): 190.5}),
+    ("g64", 16384, 2048, 32, {(1, 2, 4, 2, 16, 4, 1): 20.3, (1, 1, 4, 4, 33, 8, 2): 20.6, (1, 1, 2, 4, 33, 8, 2): 23.6}),
+    ("g64", 2048, 2048, 256, {(1, 2, 4, 2, 16, 4, 1): 18.4, (1, 2, 2, 2, 16, 4, 1): 19.3, (1, 1, 2, 4, 33, 8, 2): 21.2}),
+    ("g64", 1280, 3328, 176, {(1, 2, 4, 2, 16, 4, 1): 19.0, (1, 1, 4, 4, 33, 8, 2): 20.6}),
+]
+
+
+@pytest.mark.parametrize("fmt,m,k,n,us", MEASURED)
+def test_choice_takes_a_fast_launch(fmt, m, k, n, us):
+    """Within 3 % (the spread of repeated measurements) of the fastest launch measured there."""
+    out = (C.c_int * 7)()
+    L.lib()._ZN2sv11gemm_choiceEjbjjjPi(L.FMT_BF16 if fmt == "bf16" else L.FMT_I8, C.c_bool(fmt == "g64"), n, m, k, out)
+    assert us.get(tuple(out), 1e9) <= 1.03 * min(us.values()), f"{tuple(out)}: {us}"

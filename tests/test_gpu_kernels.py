@@ -744,7 +744,8 @@ def test_matmul_head_many_cells(gpu):
 @pytest.mark.parametrize("fmt,m,k,n", [("i8", 16384, 2048, 576), ("i8", 16384, 2048, 1152), ("bf16", 16384, 2048, 1100),
                                        ("i8", 2048, 8192, 128), ("i8", 2048, 8192, 1409), ("bf16", 2048, 8192, 768),
                                        ("i8", 3072, 2048, 704), ("bf16", 32000, 2048, 150), ("bf16", 32000, 2048, 300),
-                                       ("bf16", 32000, 2048, 577), ("g64", 6656, 1280, 600), ("g64", 1280, 3328, 1500)])
+                                       ("bf16", 32000, 2048, 577), ("g64", 6656, 1280, 600), ("g64", 1280, 3328, 1500),
+                                       ("bf16", 3072, 2048, 352), ("bf16", 32000, 2048, 161), ("g64", 16384, 2048, 33)])
 def test_matmul_built_in_choice(gpu, fmt, m, k, n):
     """The built-in launch at row counts between and past the blocks' sizes (one and several rounds of
     blocks, k splits, the 16-wide blocks of 64 and 80 tokens with bf16), with the workspace that the
