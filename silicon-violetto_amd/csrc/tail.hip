@@ -82,6 +82,16 @@ __device__ __forceinline__ void better(float& bv, uint32_t& bi, float v, uint32_
 // before t, in 32 serial runs of 32 then their bases in order. The runs sit 33 words apart in
 // LDS, so the 32 serial lanes read 32 different banks and half a run is in registers before its
 // dependent additions start; the bases are added by the same wave from its own registers.
+// upto[l] = (..(v[0] + v[1]) + ..) + v[l] over the lanes in order: after i passes of "the lane below's sum
+// plus mine" lanes 0 .. i - 1 hold theirs, added in that order. One instruction a pass; a lane's mask
+// and a register per lane would be 64 of each, which the compiler hoists and spills.
+template <int N>
+__device__ __forceinline__ void wave_sums(float& upto, float v) {
+#pragma unroll
+  for (int i = 0; i < N; i++)
+    upto = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(upto), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+}
+
 struct Scan1024 {
   float run[SV_SAMPLE_THREADS + 32];  // [32][33]: exclusive sums inside each run
   float base[33];                     // each run's base, then the total
@@ -106,14 +116,10 @@ struct Scan1024 {
           }
         }
       }
-      float b = 0.0f, mine = 0.0f;
-#pragma unroll
-      for (int g = 0; g < 32; g++) {
-        mine = tid == (uint32_t)g ? b : mine;
-        b += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), g));
-      }
-      if (tid < 32) base[tid] = mine;
-      if (tid == 0) base[32] = b;
+      float b = 0.0f;
+      wave_sums<32>(b, acc);
+      if (tid < 32) base[tid + 1] = b;
+      if (tid == 0) base[0] = 0.0f;
     }
     __syncthreads();
   }
@@ -141,9 +147,15 @@ __device__ __forceinline__ float exp2_le0(float x) {
 // One compute unit serves a row, so a row's passes are bound by its loads' latency and, at a
 // temperature, by the exponentials' VALU work (15 instructions an id: 15 us of 151680). Every
 // pass takes the ids past the cached ones in batches of BATCH loads, and a drawn share's ids are
-// evaluated by a whole wave at once with only their additions serial. MI355X, 32 rows of 151680
-// ids at T 0.6, top-p 0.95: 72 us (172 with one load at a time, a walk by one thread and the
-// scan's runs on two LDS banks); one greedy row 14 us (49); 5 greedy rows of 32000 4.8 us (7.1).
+// evaluated by a whole wave at once with only their additions serial. MI355X, launches of a graph,
+// 32 rows of 151680 ids with twelve likely ones at T 0.6, top-p 0.95: 48 us (128 with one load at a
+// time, a walk by one thread and the scan's runs on two LDS banks; 54 with a register and a lane mask
+// per lane of the walk); greedy 15 us (29); 5 greedy rows of 32000 7.2 us (9.3).
+//
+// CACHED: the logits of a thread that are kept in registers; MORE: the vocabulary has ids past them.
+// Few of them are few instructions, and without MORE nothing spills: 32 rows of 1000 ids at T 1 take
+// 8.4 us with CACHED 4 (14.5 in the kernel for any vocabulary, 9.6 with one load at a time).
+template <int CACHED, bool MORE>
 __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const sv_sample_row* rows, uint32_t* out,
                                                       const uint32_t* meta, uint32_t vocab) {
   __shared__ Scan1024 sc;
@@ -152,18 +164,18 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
   __shared__ uint32_t owner, pick;
   __shared__ float pick_x;
   constexpr uint32_t TOPS = 8;
-  __shared__ float top[TOPS][SV_SAMPLE_THREADS];
+  __shared__ float top[MORE ? TOPS : 1][MORE ? SV_SAMPLE_THREADS : 1];
   const uint32_t r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const sv_sample_row row = rows[r];
   const uint32_t pos = row.tok == SV_NO_TOK ? row.pos : meta[2 * row.tok + 1] + 1;
   const float* x = logits + (size_t)r * vocab;
 
-  // The first SAMPLE_CACHED logits of this thread (ids tid, tid + 1024, ...) are requested
+  // The first CACHED logits of this thread (ids tid, tid + 1024, ...) are requested
   // together and kept in registers; ids past that are read BATCH at a time. Every load is
   // unconditional: one lane offset, a scalar one per load, and past the vocabulary the buffer's
   // range check, whose zeros become -inf, which no pass counts.
-  constexpr int SAMPLE_CACHED = 32, BATCH = 16;
-  constexpr uint32_t NT = SV_SAMPLE_THREADS, REST = SAMPLE_CACHED * NT;
+  constexpr int BATCH = 16;
+  constexpr uint32_t NT = SV_SAMPLE_THREADS, REST = CACHED * NT;
   const float ninf = -__builtin_inff();
   // id i0 + k of the row, i0 (below the vocabulary) the same for every lane, k < 64 Ki
   auto at = [&](uint32_t i0, uint32_t k) {
@@ -172,9 +184,9 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
     const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, k * 4, 0, 0));
     return k < left ? v : ninf;
   };
-  float xc[SAMPLE_CACHED];
+  float xc[CACHED];
 #pragma unroll
-  for (int j = 0; j < SAMPLE_CACHED; j++) xc[j] = at(0, j * NT + tid);
+  for (int j = 0; j < CACHED; j++) xc[j] = at(0, j * NT + tid);
   // fn(logit, id) over the thread's BATCH ids from i0 + tid on
   auto batch = [&](uint32_t i0, auto fn) {
     float xb[BATCH];
@@ -192,11 +204,11 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
     tok = up ? i : tok;
   };
 #pragma unroll
-  for (int j = 0; j < SAMPLE_CACHED; j++) upper(xc[j], tid + j * NT);
+  for (int j = 0; j < CACHED; j++) upper(xc[j], tid + j * NT);
   // The largest logit of each of the thread's first TOPS batches, in its own LDS words: a later
   // pass over the ids above some logit reads only the batches that hold one (a row's few likely
   // ids leave nearly every batch unread).
-  for (uint32_t i0 = REST, b = 0; i0 < vocab; i0 += BATCH * NT, b++) {
+  for (uint32_t i0 = REST, b = 0; MORE && i0 < vocab; i0 += BATCH * NT, b++) {
     float t = ninf;
     batch(i0, [&](float v, uint32_t i) {
       upper(v, i);
@@ -225,9 +237,14 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
     const float c = LOG2E_F / row.temperature;
     float s = 0.0f;
     auto add = [&](float v, uint32_t) { s += exp2_le0((v - lmax) * c); };
+    // fn over the cached ids, in groups that a vocabulary of fewer ids leaves out (all 32 take 3 us)
+    auto cached = [&](auto fn) {
 #pragma unroll
-    for (int j = 0; j < SAMPLE_CACHED; j++) add(xc[j], 0);
-    for (uint32_t i0 = REST; i0 < vocab; i0 += BATCH * NT) batch(i0, add);
+      for (int j = 0; j < CACHED; j++)
+        if (MORE || j / 8 * 8 * NT < vocab) fn(xc[j], 0);
+    };
+    cached(add);
+    for (uint32_t i0 = REST; MORE && i0 < vocab; i0 += BATCH * NT) batch(i0, add);
     sc.scan(s, tid);
     const float z = sc.base[32];
     float low = ninf;
@@ -250,16 +267,20 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
         float nx = at(o, lane * NT);
         for (uint32_t i0 = o;; i0 += 64 * NT) {
           const float xi = nx;
-          const bool more = vocab - i0 > 64 * NT;
+          const bool more = MORE && vocab - i0 > 64 * NT;
           if (more) nx = at(i0 + 64 * NT, lane * NT);  // the next 64, while these are added
           const float e = xi > low ? exp2_le0((xi - lmax) * c) : 0.0f;
+          const float v = lane == 0 ? acc + e : e;
           float upto = 0.0f;
-#pragma unroll
-          for (int l = 0; l < 64; l++) {
-            acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), l));
-            upto = lane == (uint32_t)l ? acc : upto;
+          // in groups of 8 lanes: none past the share's last id or the sum that passes the offset
+          const uint64_t live = __ballot(e > 0.0f);
+          uint64_t past = 0;
+          for (uint32_t h = 8; !past && h <= (CACHED < 32 ? 8 : MORE ? 64 : 32); h += 8) {
+            wave_sums<8>(upto, v);
+            past = __ballot(off < upto) & live & (~0ull >> (64 - h));
+            if (vocab - i0 <= h * NT) break;
           }
-          const uint64_t live = __ballot(e > 0.0f), past = __ballot(off < upto) & live;
+          acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(upto), 63));
           if (live) {
             const int l = past ? __builtin_ctzll(past) : 63 - __builtin_clzll(live);
             j = i0 + l * NT;
@@ -284,9 +305,8 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float* logits, const
       auto above = [&](float v, uint32_t) {
         if (v > xj) qs += exp2_le0((v - lmax) * c);
       };
-#pragma unroll
-      for (int q = 0; q < SAMPLE_CACHED; q++) above(xc[q], 0);
-      for (uint32_t i0 = REST, b = 0; i0 < vocab; i0 += BATCH * NT, b++)
+      cached(above);
+      for (uint32_t i0 = REST, b = 0; MORE && i0 < vocab; i0 += BATCH * NT, b++)
         if (b >= TOPS || top[b][tid] > xj) batch(i0, above);
       sc.scan(qs, tid);
       if (sc.base[32] < row.top_p * z) {
@@ -788,7 +808,10 @@ sv_status sample_launch(hipStream_t stream, const float* logits, const sv_sample
   if (!logits || !rows || !out) return fail(SV_ERR_ARG, "sample: null pointer");
   if (n_rows == 0) return SV_OK;
   if (vocab == 0) return fail(SV_ERR_ARG, "sample: empty vocabulary");
-  launch(sample_kernel, dim3(n_rows), dim3(SV_SAMPLE_THREADS), 0, stream, logits, rows, out, meta, vocab);
+  const dim3 grid(n_rows), wg(SV_SAMPLE_THREADS);
+  if (vocab <= 4 * SV_SAMPLE_THREADS) launch(sample_kernel<4, false>, grid, wg, 0, stream, logits, rows, out, meta, vocab);
+  else if (vocab <= 32 * SV_SAMPLE_THREADS) launch(sample_kernel<32, false>, grid, wg, 0, stream, logits, rows, out, meta, vocab);
+  else launch(sample_kernel<32, true>, grid, wg, 0, stream, logits, rows, out, meta, vocab);
   return check_launch("sample");
 }
 

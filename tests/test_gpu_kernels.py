@@ -509,11 +509,11 @@ def test_sample_bit_exact(gpu, vocab):
     assert np.array_equal(got, ref), f"ids differ at rows {np.nonzero(got != ref)[0]}"
 
 
-@pytest.mark.parametrize("vocab", [32768, 32769, 49152, 49153, 98305])
+@pytest.mark.parametrize("vocab", [63, 1025, 4096, 4097, 8193, 32768, 32769, 49152, 49153, 98305])
 def test_sample_bit_exact_past_cached(gpu, vocab):
-    """Vocabularies around the ids a thread keeps in registers (32 x 1024) and its later batches
-    (16 x 1024): trained-like rows (a few high logits, so top-p takes several rounds), and rows of
-    infinities and NaN. Bit for bit against the oracle."""
+    """Vocabularies around the ids a thread keeps in registers (4 x 1024 or 32 x 1024, in groups of
+    8 x 1024) and its later batches (16 x 1024): trained-like rows (a few high logits, so top-p takes
+    several rounds), and rows of infinities and NaN. Bit for bit against the oracle."""
     banner(f"sample past cached vocab={vocab}")
     rng = np.random.default_rng(vocab)
     n = 32
