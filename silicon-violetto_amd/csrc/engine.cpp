@@ -490,14 +490,20 @@ struct sv_engine {
   // kv.rs:49-56 reserve(): pages until the slot holds `len` positions; the page table entries go to
   // the device from pinned memory. The caller has waited for the stream before (an earlier copy may
   // still read the same rows) and waits for it, or launches the step behind it, afterwards.
+  // Pages taken before the pool ran out stay the slot's, so their entries go up too.
   sv_status reserve(uint32_t slot, uint32_t len) {
     auto& pg = pages[slot];
     const size_t before = pg.size();
-    while (((size_t)pg.size() << cfg.page_shift) < len) {
-      if (free_pages.empty()) return fail(SV_ERR_CAPACITY, "global KV pool exhausted");
-      if (pg.size() >= max_pages) return fail(SV_ERR_CAPACITY, "sequence needs more than %u pages", max_pages);
-      pg.push_back(free_pages.back());
-      free_pages.pop_back();
+    sv_status st = SV_OK;
+    while (st == SV_OK && ((size_t)pg.size() << cfg.page_shift) < len) {
+      if (free_pages.empty()) {
+        st = fail(SV_ERR_CAPACITY, "global KV pool exhausted");
+      } else if (pg.size() >= max_pages) {
+        st = fail(SV_ERR_CAPACITY, "sequence needs more than %u pages", max_pages);
+      } else {
+        pg.push_back(free_pages.back());
+        free_pages.pop_back();
+      }
     }
     if (pg.size() > before) {
       // (the stream is idle: no earlier copy still reads the pinned rows)
@@ -505,7 +511,7 @@ struct sv_engine {
       memcpy(host_table + at, pg.data() + before, words * 4);
       SV_HIP(hipMemcpyAsync(page_table + at, host_table + at, words * 4, hipMemcpyHostToDevice, stream), "page table");
     }
-    return SV_OK;
+    return st;
   }
 
   sv_status ensure_ws(size_t bytes) {

@@ -666,6 +666,26 @@ def test_step_from_weight_file(gpu, tmp_path, group):
     wf.close()
 
 
+def test_page_table_after_exhausted_pool(gpu):
+    """A step refused because the pool ran out keeps the pages it had taken; their table entries must
+    be on the device when the sequence goes on after another one has given its pages back."""
+    banner("page table after an exhausted pool")
+    shape = ModelShape(n_layers=1)
+    eng = Engine(shape, max_seqs=2, max_step_tokens=128, max_seq_len=256, kv_tokens=128)
+    eng.set_model(SyntheticModel.generate(shape, seed=0, device="cuda"))
+    a, b = eng.new_seq(), eng.new_seq()
+    eng.bench_fill(a, 64)
+    eng.bench_fill(b, 32)                       # 6 of 8 pages of 16
+    with pytest.raises(L.SvError, match="exhausted"):
+        eng.bench_fill(a, 64)                   # takes both pages left, needs four
+    eng.free_seq(b)
+    eng.bench_fill(a, 64)
+    pages = eng.seq_pages(a)
+    table = eng.view("d_page_table", (2, eng.buf.max_pages)).cpu().numpy()
+    eng.close()
+    assert len(pages) == 8 and list(table[a, :8]) == pages
+
+
 def test_prompt_chunks_then_verify(gpu):
     """The chunk path (encode.rs:300-355): three streams on shuffled pages with 100, 37 and 500
     cached tokens each take a prompt chunk of 40, 100 and 23 tokens in one step (attention in
