@@ -123,7 +123,7 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
 
 // gemm_pipe.hip: whether mm_pipe is built for this shape (32-row tiles per wave rt, 32-token
 // tiles nt, chunks per iteration cpi), and its launch over nwg workgroups of 8 waves.
-bool gemm_pipe_built(int rt, int nt, int cpi);
+bool gemm_pipe_built(bool grouped, int rt, int nt, int cpi);
 void gemm_pipe_launch(hipStream_t stream, uint32_t fmt, bool grouped, int rt, int nt, int cpi, const MMParams& p,
                       uint32_t nwg, uint32_t n_tblk);
 

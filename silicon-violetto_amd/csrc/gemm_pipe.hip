@@ -342,9 +342,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-bool gemm_pipe_built(int rt, int nt, int cpi) {
+// With scale groups the 512-row blocks of 64 and 128 tokens hold two sets of sums, and spill: not built.
+bool gemm_pipe_built(bool grouped, int rt, int nt, int cpi) {
   return (rt == 1 && ((nt == 1 && cpi == 2) || (nt == 2 && cpi == 2) || (nt == 4 && cpi == 1))) ||
-         (rt == 2 && ((nt == 1 && cpi == 1) || (nt == 2 && cpi == 1) || (nt == 4 && cpi == 1)));
+         (rt == 2 && cpi == 1 && (nt == 1 || (!grouped && (nt == 2 || nt == 4))));
 }
 
 void gemm_pipe_launch(hipStream_t stream, uint32_t fmt, bool grouped, int rt, int nt, int cpi, const MMParams& p,
@@ -354,13 +355,13 @@ void gemm_pipe_launch(hipStream_t stream, uint32_t fmt, bool grouped, int rt, in
     launch((mm_pipe<F, R, N, C, G>), dim3(nwg), dim3(512), 0, stream, p, n_tblk);      \
     return;                                                                            \
   }
-#define SV_PIPE_F(F, G) SV_PIPE(F, 1, 1, 2, G) SV_PIPE(F, 1, 2, 2, G) SV_PIPE(F, 1, 4, 1, G) SV_PIPE(F, 2, 1, 1, G) SV_PIPE(F, 2, 2, 1, G) SV_PIPE(F, 2, 4, 1, G)
+#define SV_PIPE_F(F, G) SV_PIPE(F, 1, 1, 2, G) SV_PIPE(F, 1, 2, 2, G) SV_PIPE(F, 1, 4, 1, G) SV_PIPE(F, 2, 1, 1, G)
   if (fmt != SV_FMT_I8) {
-    SV_PIPE_F(SV_FMT_BF16, false)
+    SV_PIPE_F(SV_FMT_BF16, false) SV_PIPE(SV_FMT_BF16, 2, 2, 1, false) SV_PIPE(SV_FMT_BF16, 2, 4, 1, false)
   } else if (grouped) {
     SV_PIPE_F(SV_FMT_I8, true)
   } else {
-    SV_PIPE_F(SV_FMT_I8, false)
+    SV_PIPE_F(SV_FMT_I8, false) SV_PIPE(SV_FMT_I8, 2, 2, 1, false) SV_PIPE(SV_FMT_I8, 2, 4, 1, false)
   }
 #undef SV_PIPE_F
 #undef SV_PIPE

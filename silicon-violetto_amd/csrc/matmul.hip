@@ -18,8 +18,8 @@
 //     scheduling.
 //   - The sum of squares of X for the folded rms-norm (EPI_NORM/SWIGLU, NORM_IN) rides
 //     along the same path.
-// int8 weights need one scale per k chunk: groups of 256 or more, or one scale per row
-// (per-output-channel, any k).
+// int8 weights: the skinny kernels take one scale per k chunk (groups of 256 or more, or one per row),
+// the one-shot kernel and the GEMMs groups of 64 and more.
 #include "gemm_device.h"
 
 #include <algorithm>
@@ -866,33 +866,30 @@ __global__ __launch_bounds__(256) void mm_gemm(MMParams p, uint32_t n_tblk) {
   }
 }
 
-// 32 x 32 x 16 GEMM (n > 16 rows). gfx950 runs v_mfma_f32_32x32x16_bf16 (32,768 flops) in
-// about the time v_mfma_f32_16x16x32_bf16 (16,384 flops) takes when both stream back to back
-// (measured: 2.2 vs 1.2 PFLOP/s), so the 32-wide tile halves the matrix-core time of the same
-// product. Same structure as mm_gemm: NW waves (4 or 8), BM = 32 RT NW rows (RT 32-row tiles per wave),
-// BN = 32 NT tokens, 1/S of k, chunks of 64 k in a software pipeline GD deep, X split once per
-// workgroup into LDS, k splits merged by the last split to arrive.
+// 32 x 32 x 16 GEMM of int8 weights with a scale per row in blocks of 256 x 32. gfx950 runs
+// v_mfma_f32_32x32x16_bf16 (32,768 flops) in about the time v_mfma_f32_16x16x32_bf16 (16,384 flops) takes
+// when both stream back to back (measured: 2.2 vs 1.2 PFLOP/s), so the 32-wide tile halves the matrix-core
+// time of the same product. Same structure as mm_gemm: 8 waves, BM = 256 (a 32-row tile per wave), BN = 32
+// tokens, 1/S of k, chunks of 64 k in a software pipeline GD = 4 deep, X split once per workgroup into
+// LDS, k splits merged by the last split to arrive. Where that block is the fastest, its 64-k steps beat
+// the two phases of mm_pipe's block of the same size: qkv, 3072 x 2048, at 512 rows 20.3 us against 24.1,
+// down, 2048 x 8192, at 160 rows 25.2 against 27.2, gate_up, 16384 x 2048, at 96 rows 23.3 against 24.8.
 //   - MFMA lane (c, h) = (lane % 32, lane / 32) supplies A row c and B column c with 8 k per
 //     step; the chunk's k order is permuted (the same way for A and B): step ks, lane half h,
 //     element e is k = 32 h + 8 ks + e. So a lane's weights for a chunk are 32 consecutive k of
-//     its row: two 16-byte words (bf16: four) of the tiled layout, word q = 2 h + qq of the
-//     lane's 16-row block.
+//     its row: two 16-byte words of the tiled layout, word q = 2 h + qq of the lane's 16-row block.
 //   - X in LDS as [hi, lo][4 steps][2 halves][32 columns] 16-byte slots, the column XOR-ed
 //     with 4 h + ks (< 8): reads of a quarter-wave start at a multiple of 16 slots and keep the
 //     slot order up to a permutation within 8 lanes, writes of a token's 8 k groups land on 8
 //     different slots mod 8 (both conflict-free on gfx950).
 //   - Lane (c, h) receives rows 8 j + 4 h + i (j, i = 0..3) of token c: f32x4 row groups, so
 //     the epilogue (rms-norm fold, SwiGLU pairs, residual) is the 16-wide one per group.
-template <int FMT, int RT, int NT, int GD, int NW, int CPI>
-__global__ __launch_bounds__(NW * 64) void mm_gemm32(MMParams p, uint32_t n_tblk) {
-  static_assert(GD % (2 * CPI) == 0, "iteration parity = buffer parity");
-  constexpr int BN = 32 * NT;
-  constexpr int ESZ = FMT == SV_FMT_I8 ? 1 : 2;
-  constexpr int WL = FMT == SV_FMT_I8 ? 1 : 2;  // 16-byte words per lane per 16 k
-  constexpr int NTH = NW * 64;
-  constexpr int PAIRS = BN * 8;                 // (token, 8-k group) pairs per chunk
-  constexpr int PPT = (PAIRS + NTH - 1) / NTH;  // pairs per thread
-  __shared__ u32x4 xs[2][CPI][NT][2][256];  // [buffer][chunk of the iteration]
+//   - Two accumulator sets (even and odd k steps) halve the chain of dependent products, and every B
+//     operand of a chunk is requested before the first product (one LDS wait per chunk).
+__global__ __launch_bounds__(512) void mm_gemm32(MMParams p, uint32_t n_tblk) {
+  constexpr int BN = 32, GD = 4;
+  constexpr uint32_t OOB = 0x80000000u;
+  __shared__ u32x4 xs[2][2][256];  // [buffer][hi, lo]
   __shared__ float ssp[BN][8];
   __shared__ uint32_t last_flag;
   const int tid = threadIdx.x, lane = tid & 63, c32 = lane & 31, h = lane >> 5;
@@ -905,273 +902,154 @@ __global__ __launch_bounds__(NW * 64) void mm_gemm32(MMParams p, uint32_t n_tblk
   uint32_t tblk, sp, rblk;
   gemm_item(item, n_tblk, S, nwg / (n_tblk * S), p.order, tblk, sp, rblk);
   const uint32_t t0 = tblk * BN;
-  const uint32_t row0 = (rblk * NW + wv) * 32 * RT;  // this wave's first row
+  const uint32_t row0 = (rblk * 8 + wv) * 32;  // this wave's first row
   const uint32_t nc = __builtin_amdgcn_readfirstlane(p.k / GKC / S);
   const uint32_t cb = __builtin_amdgcn_readfirstlane(sp * nc);
 
   const __amdgpu_buffer_rsrc_t xrs = coherent_rsrc(p.x), wrs = coherent_rsrc(p.w);
-  constexpr uint32_t OOB = 0x80000000u;
-  // Weights: lane (c, h) takes row c of the wave's 32-row tile r (16-row block c / 16, row
-  // c % 16), words q = 2 h, 2 h + 1 of each chunk.
-  const uint32_t tile_bytes = 16 * p.k * ESZ;  // one 16-row block over all k
+  // Weights: lane (c, h) takes row c of the wave's tile (16-row block c / 16, row c % 16), words
+  // q = 2 h, 2 h + 1 of each chunk.
+  const uint32_t tile_bytes = 16 * p.k;  // one 16-row block over all k
   const uint32_t wl = p.tiled ? (uint32_t)(c32 >> 4) * tile_bytes + (uint32_t)((c32 & 15) + 32 * h) * 16
-                              : ((uint32_t)c32 * p.k + 32 * h) * ESZ;
-  const uint32_t chunk_bytes = p.tiled ? 1024 * ESZ : 64 * ESZ, qq_bytes = p.tiled ? 256 : 16 * ESZ,
-                 v_bytes = p.tiled ? 1024 : 16;
-  uint32_t xoff[PPT];
-#pragma unroll
-  for (int j = 0; j < PPT; j++) {
-    const int i = tid + NTH * j;
-    const uint32_t tt = t0 + i / 8;
-    xoff[j] = i < PAIRS && tt < p.n ? ((p.x_rows ? p.x_rows[tt] : tt) * p.k + 8 * (i % 8)) * 4 : OOB;
-  }
-  auto load_x = [&](uint32_t c, f32x4 (&xr)[PPT][2]) {
+                              : (uint32_t)c32 * p.k + 32 * h;
+  const uint32_t chunk_bytes = p.tiled ? 1024 : 64, qq_bytes = p.tiled ? 256 : 16;
+  const uint32_t rbase = p.tiled ? row0 / 16 * tile_bytes : row0 * p.k;
+  // X: threads 0-255 take 8 k of a token each.
+  const int tok = tid / 8, g8 = tid % 8;  // k group g8 = 4 h + ks
+  const uint32_t tt = t0 + tok;
+  const uint32_t xoff = tok < BN && tt < p.n ? ((p.x_rows ? p.x_rows[tt] : tt) * p.k + 8 * g8) * 4 : OOB;
+  const int xslot = 64 * (g8 & 3) + 32 * (g8 >> 2) + ((tok & 31) ^ g8);
+  auto load_x = [&](uint32_t c, f32x4 (&xr)[2]) {
     const uint32_t so = __builtin_amdgcn_readfirstlane((cb + min(c, nc - 1)) * GKC * 4);
-#pragma unroll
-    for (int j = 0; j < PPT; j++) {
-      const uint32_t vo = c < nc ? xoff[j] : OOB;
-      xr[j][0] = __builtin_bit_cast(f32x4, buf_ld16(xrs, vo, so));
-      xr[j][1] = __builtin_bit_cast(f32x4, buf_ld16(xrs, vo + 16, so));
-    }
+    const uint32_t vo = c < nc ? xoff : OOB;
+    xr[0] = __builtin_bit_cast(f32x4, buf_ld16(xrs, vo, so));
+    xr[1] = __builtin_bit_cast(f32x4, buf_ld16(xrs, vo + 16, so));
   };
-  auto load_w = [&](uint32_t c, u32x4 (&wr)[RT][2 * WL]) {
+  auto load_w = [&](uint32_t c, u32x4 (&wr)[2]) {
     const uint32_t cc = c < nc ? cb + c : 0u;
     const uint32_t vo = c < nc ? wl : OOB;
 #pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-      for (int qq = 0; qq < 2; qq++)
-#pragma unroll
-        for (int v = 0; v < WL; v++) {
-          const uint32_t rbase = p.tiled ? (row0 / 16 + 2 * r) * tile_bytes : (row0 + 32 * r) * p.k * ESZ;
-          wr[r][qq * WL + v] =
-              buf_ld16(wrs, vo, __builtin_amdgcn_readfirstlane(rbase + cc * chunk_bytes + qq * qq_bytes + v * v_bytes));
-        }
+    for (int qq = 0; qq < 2; qq++)
+      wr[qq] = buf_ld16(wrs, vo, __builtin_amdgcn_readfirstlane(rbase + cc * chunk_bytes + qq * qq_bytes));
   };
-  float ssacc[PPT];
+  float ssacc = 0.0f;
+  auto store_x = [&](int buf, const f32x4 (&xr)[2]) {
+    if (tok >= BN) return;
+    float v[8];
 #pragma unroll
-  for (int j = 0; j < PPT; j++) ssacc[j] = 0.0f;
-  auto store_x = [&](int buf, int u, const f32x4 (&xr)[PPT][2]) {
-#pragma unroll
-    for (int j = 0; j < PPT; j++) {
-      const int i = tid + NTH * j;
-      if (PAIRS % NTH != 0 && i >= PAIRS) continue;
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[e] = xr[j][0][e];
-        v[4 + e] = xr[j][1][e];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; e++) ssacc[j] = __builtin_fmaf(v[e], v[e], ssacc[j]);
-      bf16x8 hv, lv;
-      split8(v, hv, lv);
-      const int tok = i / 8, g8 = i % 8;  // k group g8 = 4 h + ks
-      const int slot = 64 * (g8 & 3) + 32 * (g8 >> 2) + ((tok & 31) ^ g8);
-      xs[buf][u][tok >> 5][0][slot] = __builtin_bit_cast(u32x4, hv);
-      xs[buf][u][tok >> 5][1][slot] = __builtin_bit_cast(u32x4, lv);
+    for (int e = 0; e < 4; e++) {
+      v[e] = xr[0][e];
+      v[4 + e] = xr[1][e];
     }
+#pragma unroll
+    for (int e = 0; e < 8; e++) ssacc = __builtin_fmaf(v[e], v[e], ssacc);
+    bf16x8 hv, lv;
+    split8(v, hv, lv);
+    xs[buf][0][xslot] = __builtin_bit_cast(u32x4, hv);
+    xs[buf][1][xslot] = __builtin_bit_cast(u32x4, lv);
   };
 
-  // One tile per wave: two accumulator sets (even and odd k-steps) halve the chain of
-  // dependent products, and every B operand of an iteration is requested before the first
-  // product (one LDS wait per iteration). Wider waves have independent tiles to interleave and
-  // read each k-step's operands as they go (fewer registers).
-  constexpr bool DUAL = RT * NT == 1, UPF = NT == 1;
-  f32x16 acc[RT][NT], acc2[1][1];  // acc2: used when DUAL
+  f32x16 acc[2];
 #pragma unroll
-  for (int r = 0; r < RT; r++)
+  for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[r][n][e] = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 16; e++) acc2[0][0][e] = 0.0f;
+    for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
 
-  f32x4 xr[GD][PPT][2];
-  u32x4 wr[GD][RT][2 * WL];
+  f32x4 xr[GD][2];
+  u32x4 wr[GD][2];
 #pragma unroll
   for (int d = 0; d < GD; d++) {
     load_w(d, wr[d]);
     load_x(d, xr[d]);
   }
-#pragma unroll
-  for (int u = 0; u < CPI; u++) {
-    store_x(0, u, xr[u]);
-    load_x(GD + u, xr[u]);
-  }
+  store_x(0, xr[0]);
+  load_x(GD, xr[0]);
   lds_barrier();
 
-  // CPI chunks per barrier: chunks c .. c + CPI - 1 multiplied from LDS buffer `buf` while
-  // chunks c + CPI .. are split into the other.
+  // Chunk c multiplied from LDS buffer `buf` while chunk c + 1 is split into the other.
   for (uint32_t c0 = 0; c0 < nc; c0 += GD) {
 #pragma unroll
-    for (int d = 0; d < GD; d += CPI) {
+    for (int d = 0; d < GD; d++) {
       const uint32_t c = c0 + d;
-      const int buf = (d / CPI) & 1;
-      u32x4 cur[CPI][RT][2 * WL];
+      const int buf = d & 1, dn = (d + 1) % GD;
+      const u32x4 cur[2] = {wr[d][0], wr[d][1]};
+      load_w(c + GD, wr[d]);
+      bf16x8 bx[4][2];
 #pragma unroll
-      for (int u = 0; u < CPI; u++) {
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-          for (int v = 0; v < 2 * WL; v++) cur[u][r][v] = wr[d + u][r][v];
-        load_w(c + u + GD, wr[d + u]);
-      }
-      auto read_b = [&](int u, int ks, bf16x8 (&bk)[NT][2]) {
+      for (int ks = 0; ks < 4; ks++) {
         const int slot = 64 * ks + 32 * h + (c32 ^ (4 * h + ks));
 #pragma unroll
-        for (int n = 0; n < NT; n++)
-#pragma unroll
-          for (int hl = 0; hl < 2; hl++) bk[n][hl] = __builtin_bit_cast(bf16x8, xs[buf][u][n][hl][slot]);
-      };
-      bf16x8 bx[CPI][UPF ? 4 : 1][NT][2];
-      if constexpr (UPF) {
-#pragma unroll
-        for (int u = 0; u < CPI; u++)
-#pragma unroll
-          for (int ks = 0; ks < 4; ks++) read_b(u, ks, bx[u][ks]);
+        for (int hl = 0; hl < 2; hl++) bx[ks][hl] = __builtin_bit_cast(bf16x8, xs[buf][hl][slot]);
       }
       __builtin_amdgcn_sched_barrier(0);
-      // The next iteration's X (requested GD - CPI chunks ago) to the other buffer while this
-      // iteration's operands arrive, then the chunks GD further requested into its registers:
-      // the split's VALU work overlaps the LDS reads' latency, and the products the writes'.
-#pragma unroll
-      for (int u = 0; u < CPI; u++) {
-        const int dn = (d + CPI + u) % GD;
-        store_x(buf ^ 1, u, xr[dn]);
-        load_x(c + CPI + u + GD, xr[dn]);
-      }
+      // The next chunk's X (requested GD - 1 chunks ago) to the other buffer while this chunk's
+      // operands arrive, then the chunk GD further requested into its registers: the split's VALU
+      // work overlaps the LDS reads' latency, and the products the writes'.
+      store_x(buf ^ 1, xr[dn]);
+      load_x(c + 1 + GD, xr[dn]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < CPI; u++)
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-          bf16x8 a[RT];
-#pragma unroll
-          for (int r = 0; r < RT; r++) {
-            if (FMT == SV_FMT_I8) {
-              const u32x4 w = cur[u][r][ks >> 1];
-              a[r] = i8x8_to_bf(w[2 * (ks & 1)], w[2 * (ks & 1) + 1]);
-            } else {
-              a[r] = __builtin_bit_cast(bf16x8, cur[u][r][ks]);
-            }
-          }
-          auto products = [&](const bf16x8 (&bk)[NT][2]) {
-#pragma unroll
-            for (int n = 0; n < NT; n++)
-#pragma unroll
-              for (int r = 0; r < RT; r++) {
-                f32x16& g = (DUAL && (ks & 1)) ? acc2[0][0] : acc[r][n];
-                g = mfma32(a[r], bk[n][0], g);
-                g = mfma32(a[r], bk[n][1], g);
-              }
-          };
-          if constexpr (UPF) {
-            products(bx[u][ks]);
-          } else {
-            bf16x8 bk[NT][2];
-            read_b(u, ks, bk);
-            products(bk);
-          }
-        }
+      for (int ks = 0; ks < 4; ks++) {
+        const u32x4 w = cur[ks >> 1];
+        const bf16x8 a = i8x8_to_bf(w[2 * (ks & 1)], w[2 * (ks & 1) + 1]);
+        acc[ks & 1] = mfma32(a, bx[ks][0], acc[ks & 1]);
+        acc[ks & 1] = mfma32(a, bx[ks][1], acc[ks & 1]);
+      }
       lds_barrier();
     }
   }
-  if constexpr (DUAL) acc[0][0] += acc2[0][0];
-  // Per-row int8 scales: lane (c, h) holds rows 8 j + 4 h + i of each tile.
-  if (FMT == SV_FMT_I8) {
+  f32x16 sum = acc[0] + acc[1];
+  // Row scales: lane (c, h) holds rows 8 j + 4 h + i of its tile.
 #pragma unroll
-    for (int r = 0; r < RT; r++)
+  for (int j = 0; j < 4; j++) {
+    const uint16_t* sp4 = p.scales + row0 + 8 * j + 4 * h;  // any alignment
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const uint16_t* sp4 = p.scales + row0 + 32 * r + 8 * j + 4 * h;  // any alignment
-        const float s0 = bf(ldg_u16(sp4)), s1 = bf(ldg_u16(sp4 + 1)), s2 = bf(ldg_u16(sp4 + 2)),
-                    s3 = bf(ldg_u16(sp4 + 3));
-#pragma unroll
-        for (int n = 0; n < NT; n++) {
-          acc[r][n][4 * j + 0] *= s0;
-          acc[r][n][4 * j + 1] *= s1;
-          acc[r][n][4 * j + 2] *= s2;
-          acc[r][n][4 * j + 3] *= s3;
-        }
-      }
+    for (int i = 0; i < 4; i++) sum[4 * j + i] *= bf(ldg_u16(sp4 + i));
   }
-#pragma unroll
-  for (int j = 0; j < PPT; j++) {
-    const int i = tid + NTH * j;
-    if (i < PAIRS) ssp[i / 8][i % 8] = ssacc[j];
-  }
+  if (tok < BN) ssp[tok][g8] = ssacc;
   __syncthreads();
-  float ssn[NT];
-#pragma unroll
-  for (int n = 0; n < NT; n++) {
-    const uint32_t tl = 32 * n + c32;
+  auto token_ss = [&](uint32_t tl) {
     float ss = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; e++) ss += ssp[tl][e];
-    ssn[n] = ss;
-  }
+    return ss;
+  };
+  float ss = token_ss(c32);
 
   if (S > 1) {
-    // [cell][split][NTH threads][RT NT 4] f32x4 and [cell][split][BN] sums of squares; the
-    // last split of the cell adds them in split order.
+    // [cell][split][512 threads][4] f32x4 and [cell][split][BN] sums of squares; the last split of
+    // the cell adds them in split order.
     const uint32_t cell = rblk * n_tblk + tblk;
     const __amdgpu_buffer_rsrc_t prs = coherent_rsrc(p.part), srs = coherent_rsrc(p.ssp);
-    constexpr uint32_t PER = NTH * RT * NT * 64;
+    constexpr uint32_t PER = 512 * 64;
     const uint32_t pb = (cell * S) * PER;
 #pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          store_wt4(prs, pb + sp * PER + (((r * NT + n) * 4 + j) * NTH + tid) * 16,
-                    f32x4{acc[r][n][4 * j], acc[r][n][4 * j + 1], acc[r][n][4 * j + 2], acc[r][n][4 * j + 3]});
-    for (int tt = tid; tt < BN; tt += NTH)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ssp[tt][0] + ssp[tt][1] + ssp[tt][2] + ssp[tt][3] +
-                                                            ssp[tt][4] + ssp[tt][5] + ssp[tt][6] + ssp[tt][7]),
-                                            srs, ((cell * S + sp) * BN + tt) * 4, 0, SV_CPOL_SC1);
+    for (int j = 0; j < 4; j++)
+      store_wt4(prs, pb + sp * PER + (j * 512 + tid) * 16, f32x4{sum[4 * j], sum[4 * j + 1], sum[4 * j + 2], sum[4 * j + 3]});
+    if (tid < BN)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ss), srs, ((cell * S + sp) * BN + tid) * 4, 0, SV_CPOL_SC1);
     if (!arrive_last(p.counters + cell, S, &last_flag)) return;
 #pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) acc[r][n][e] = 0.0f;
-#pragma unroll
-    for (int n = 0; n < NT; n++) ssn[n] = 0.0f;
+    for (int e = 0; e < 16; e++) sum[e] = 0.0f;
+    ss = 0.0f;
     for (uint32_t s2 = 0; s2 < S; s2++) {
 #pragma unroll
-      for (int r = 0; r < RT; r++)
+      for (int j = 0; j < 4; j++) {
+        const f32x4 v = load_wt4(prs, pb + s2 * PER + (j * 512 + tid) * 16);
 #pragma unroll
-        for (int n = 0; n < NT; n++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const f32x4 v = load_wt4(prs, pb + s2 * PER + (((r * NT + n) * 4 + j) * NTH + tid) * 16);
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[r][n][4 * j + i] += v[i];
-          }
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-        ssn[n] += __uint_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(srs, ((cell * S + s2) * BN + 32 * n + c32) * 4, 0, SV_CPOL_SC1));
+        for (int i = 0; i < 4; i++) sum[4 * j + i] += v[i];
+      }
+      ss += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srs, ((cell * S + s2) * BN + c32) * 4, 0, SV_CPOL_SC1));
     }
   }
 
-  // Epilogue: each (tile, token tile, j) is a group of 4 rows for token t0 + 32 n + c.
+  // Epilogue: each j is a group of 4 rows for token t0 + c.
+  const uint32_t t = t0 + c32;
+  if (t >= p.n) return;
 #pragma unroll
-  for (int n = 0; n < NT; n++) {
-    const uint32_t t = t0 + 32 * n + c32;
-    if (t >= p.n) continue;
-#pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        f32x4 col[1] = {f32x4{acc[r][n][4 * j], acc[r][n][4 * j + 1], acc[r][n][4 * j + 2], acc[r][n][4 * j + 3]}};
-        gemm_epilogue<1>(p, col, row0 + 32 * r + 8 * j + 4 * h, 0, t, ssn[n],
-                         rblk == 0 && wv == 0 && r == 0 && j == 0 && h == 0);
-      }
+  for (int j = 0; j < 4; j++) {
+    f32x4 col[1] = {f32x4{sum[4 * j], sum[4 * j + 1], sum[4 * j + 2], sum[4 * j + 3]}};
+    gemm_epilogue<1>(p, col, row0 + 8 * j + 4 * h, 0, t, ss, rblk == 0 && wv == 0 && j == 0 && h == 0);
   }
 }
 
@@ -1180,8 +1058,8 @@ __global__ __launch_bounds__(NW * 64) void mm_gemm32(MMParams p, uint32_t n_tblk
 struct GemmCfg {
   int rtw, nt, s, d;  // d: chunks in flight (2, 4 or 8)
   int mf = 16;        // 16: mm_gemm (16-wide MFMA tiles), 32: mm_gemm32, 33: mm_pipe (both 32-wide)
-  int nw = 4;         // waves per workgroup (mm_gemm32: 4 or 8)
-  int cpi = 1;        // mm_gemm32: chunks per barrier (1, or 2 with 4 chunks in flight)
+  int nw = 4;         // waves per workgroup (mm_gemm32 and mm_pipe: 8)
+  int cpi = 1;        // mm_pipe: chunks per half iteration
   uint32_t tw() const { return mf == 16 ? 16u : 32u; }
   uint32_t bm() const { return (uint32_t)(nw * rtw) * tw(); }
   uint32_t bn() const { return tw() * nt; }
@@ -1302,8 +1180,9 @@ static GemmCfg pick_builtin(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
     if (c.nt == 5) c.d = 2;
     return c;
   }
-  // Below that, 256-row x 32-token blocks without splits where they still make 512 workgroups
-  // (measured on gate_up at 256 and 320 rows: 3-25% faster than 128-row blocks in splits).
+  // Below that, 256-row x 32-token blocks without splits where they make 512 workgroups: int8 of 43,776
+  // rows and more below 96 tokens, bf16 with k of 512 or less (65536 x 1024 int8 at 64 tokens 29 us, 41 in
+  // splits of 128 rows; 16384 x 512 bf16 at 256 tokens 19, 31).
   if (!grouped && m % 256 == 0 && (uint64_t)(m / 256) * ((n + 31) / 32) >= 512) return GemmCfg{4, 2, 1, 2};
   // Long reductions (k of 8192 or more): the largest row block (256, 128, 64 rows) that makes
   // 512 workgroups with four or eight k splits (measured on the down projection at 24-512
@@ -1369,19 +1248,14 @@ static size_t gemm_ws_layout(uint32_t n, uint32_t m, const GemmCfg& c, size_t* s
   return off;
 }
 
-static bool gemm_shape_ok(uint32_t m, uint32_t k, const GemmCfg& c) {
-  const bool nt_ok = c.nt == 2 || c.nt == 3 || c.nt == 4 || c.nt == 5 || c.nt == 8;
-  if (c.mf == 33)
-    return gemm_pipe_built(c.rtw, c.nt, c.cpi) && c.nw == 8 && c.s >= 1 && c.s <= 64 &&
-           m % c.bm() == 0 && (k / GKC) % c.s == 0;
-  // 32-wide tiles: one or two row tiles per wave, one to three token tiles.
+static bool gemm_shape_ok(uint32_t fmt, bool grouped, uint32_t m, uint32_t k, const GemmCfg& c) {
+  if (c.s < 1 || c.s > 64 || m % c.bm() || (k / GKC) % c.s) return false;
+  if (c.mf == 33) return c.nw == 8 && gemm_pipe_built(grouped, c.rtw, c.nt, c.cpi);
   if (c.mf == 32)
-    return (c.rtw == 1 || c.rtw == 2) && c.nt >= 1 && c.nt <= 3 && (c.d == 2 || c.d == 4) && (c.nw == 4 || c.nw == 8) &&
-           (c.cpi == 1 || (c.cpi == 2 && c.d == 4)) &&
-           c.s >= 1 && c.s <= 64 &&
-           m % c.bm() == 0 && (k / GKC) % c.s == 0;
-  return c.mf == 16 && c.nw == 4 && nt_ok && (c.rtw == 1 || c.rtw == 2 || (c.rtw == 4 && c.nt <= 5)) && (c.d == 2 || c.d == 4 || c.d == 8) && c.s >= 1 && c.s <= 64 && m % (64 * c.rtw) == 0 &&
-         (k / GKC) % c.s == 0;
+    return fmt == SV_FMT_I8 && !grouped && c.rtw == 1 && c.nt == 1 && c.d == 4 && c.nw == 8 && c.cpi == 1;
+  const bool nt_ok = c.nt == 2 || c.nt == 3 || c.nt == 4 || c.nt == 5 || c.nt == 8;
+  return c.mf == 16 && c.nw == 4 && nt_ok && (c.rtw == 1 || (!grouped && (c.rtw == 2 || (c.rtw == 4 && c.nt <= 5)))) &&
+         (c.d == 2 || c.d == 4 || c.d == 8);
 }
 
 template <int FMT, int RTW, int NT, bool GR>
@@ -1400,22 +1274,6 @@ static void gemm_dispatch_nt(hipStream_t stream, const MMParams& p, int nt, int 
     case 5: gemm_launch_one<FMT, RTW, 5, GR>(stream, p, d, nwg, n_tblk); break;
     default: gemm_launch_one<FMT, RTW, (RTW == 4 ? 5 : 8), GR>(stream, p, d, nwg, n_tblk); break;
   }
-}
-
-static void gemm_dispatch32(hipStream_t stream, uint32_t fmt, const GemmCfg& c, const MMParams& p, uint32_t nwg,
-                            uint32_t n_tblk) {
-#define SV_G32W(F, R, N, D, C)                                                                 \
-  (c.nw == 8 ? launch((mm_gemm32<F, R, N, D, 8, C>), dim3(nwg), dim3(512), 0, stream, p, n_tblk) \
-             : launch((mm_gemm32<F, R, N, D, 4, C>), dim3(nwg), dim3(256), 0, stream, p, n_tblk))
-#define SV_G32(F, R, N, D) (D == 4 && c.cpi == 2 ? SV_G32W(F, R, N, 4, 2) : SV_G32W(F, R, N, D, 1))
-#define SV_G32_NT(F, R, D) (c.nt == 1 ? SV_G32(F, R, 1, D) : c.nt == 2 ? SV_G32(F, R, 2, D) : SV_G32(F, R, 3, D))
-#define SV_G32_D(F, R) (c.d == 4 ? SV_G32_NT(F, R, 4) : SV_G32_NT(F, R, 2))
-  if (fmt == SV_FMT_I8) c.rtw == 2 ? SV_G32_D(SV_FMT_I8, 2) : SV_G32_D(SV_FMT_I8, 1);
-  else c.rtw == 2 ? SV_G32_D(SV_FMT_BF16, 2) : SV_G32_D(SV_FMT_BF16, 1);
-#undef SV_G32_D
-#undef SV_G32_NT
-#undef SV_G32
-#undef SV_G32W
 }
 
 // The work order for nrb row blocks x S splits x n_tblk token blocks with the least HBM traffic
@@ -1481,7 +1339,7 @@ static uint32_t gemm_order(uint32_t nrb, uint32_t n_tblk, uint32_t S, double w_b
 static sv_status gemm_launch(hipStream_t stream, uint32_t fmt, MMParams& p, void* ws, size_t ws_bytes) {
   const bool grouped = fmt == SV_FMT_I8 && !p.per_row;
   const GemmCfg c = pick_gemm(fmt, grouped, p.n, p.m, p.k);
-  if (!gemm_shape_ok(p.m, p.k, c) || (grouped && c.mf != 33 && (c.rtw != 1 || c.mf != 16)))
+  if (!gemm_shape_ok(fmt, grouped, p.m, p.k, c))
     return fail(SV_ERR_ARG, "matmul (gemm): launch shape rtw %d, nt %d, splits %d for m %u, k %u", c.rtw, c.nt, c.s,
                 p.m, p.k);
   if ((size_t)p.m * p.k * (fmt == SV_FMT_I8 ? 1 : 2) >= (1ull << 31) || (size_t)p.n * p.k * 4 >= (1ull << 31))
@@ -1510,7 +1368,7 @@ static sv_status gemm_launch(hipStream_t stream, uint32_t fmt, MMParams& p, void
   if (c.mf == 33) {
     gemm_pipe_launch(stream, fmt, grouped, c.rtw, c.nt, c.cpi, p, nwg, n_tblk);
   } else if (c.mf == 32) {
-    gemm_dispatch32(stream, fmt, c, p, nwg, n_tblk);
+    launch(mm_gemm32, dim3(nwg), dim3(512), 0, stream, p, n_tblk);
   } else if (fmt == SV_FMT_I8) {
     if (grouped) gemm_dispatch_nt<SV_FMT_I8, 1, true>(stream, p, c.nt, c.d, nwg, n_tblk);
     else if (c.rtw == 4) gemm_dispatch_nt<SV_FMT_I8, 4, false>(stream, p, c.nt, c.d, nwg, n_tblk);

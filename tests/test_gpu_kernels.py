@@ -780,15 +780,7 @@ def test_matmul_built_in_choice(gpu, fmt, m, k, n):
                                                   (2, 4, 2, 4), (1, 5, 4, 4), (2, 5, 1, 4), (2, 8, 2, 4), (1, 8, 1, 4),
                                                   (4, 4, 1, 4), (4, 2, 2, 4), (4, 5, 4, 4), (4, 4, 2, 2), (4, 3, 1, 2),
                                                   (4, 2, 4, 2), (4, 2, 1, 2), (2, 2, 4, 2), (1, 2, 2, 2), (2, 5, 1, 2),
-                                                  (2, 2, 8, 2), (1, 2, 8, 2), (4, 2, 8, 2),
-                                                  # 32 x 32 x 16 tiles (the fifth field: tile width)
-                                                  (1, 1, 1, 2, 32), (1, 1, 2, 2, 32), (2, 1, 4, 2, 32), (1, 2, 1, 4, 32),
-                                                  (2, 2, 2, 2, 32), (1, 3, 8, 2, 32), (2, 3, 1, 4, 32), (1, 1, 8, 4, 32),
-                                                  # eight waves (the sixth field)
-                                                  (1, 1, 2, 2, 32, 8), (1, 2, 1, 2, 32, 8), (2, 1, 4, 4, 32, 8),
-                                                  (1, 3, 8, 2, 32, 8),
-                                                  # two chunks per barrier (the seventh field)
-                                                  (1, 1, 2, 4, 32, 8, 2), (2, 1, 1, 4, 32, 4, 2), (1, 2, 8, 4, 32, 8, 2)])
+                                                  (2, 2, 8, 2), (1, 2, 8, 2), (4, 2, 8, 2)])
 @pytest.mark.parametrize("n", [17, 100, 170])
 def test_matmul_gemm_launch_shapes(gpu, shape, n):
     """Every GEMM launch shape (row tiles per wave, token tiles, k splits merged by the last
@@ -797,17 +789,15 @@ def test_matmul_gemm_launch_shapes(gpu, shape, n):
     the tiled layout, with a row gather, ragged token blocks (17, 100 rows) and a k whose chunk
     count leaves a partial round of zero chunks (k = 1280: 20 chunks; 2560 = 40 chunks for eight
     splits, five each); two calls share one workspace. The shape is forced through the
-    library's internal override: 16-wide tiles (mm_gemm) and 32-wide tiles (mm_gemm32) with 4
-    or 8 waves and one or two chunks per barrier."""
-    rtw, nt, splits, depth, mf, nw, cpi = (tuple(shape) + (16, 4, 1)[len(shape) - 4:])[:7]
-    banner(f"gemm launch shape rtw={rtw} nt={nt} splits={splits} depth={depth} tile={mf} waves={nw} "
-           f"chunks per barrier={cpi} n={n}")
+    library's internal override (mm_gemm's)."""
+    rtw, nt, splits, depth = shape
+    banner(f"gemm launch shape rtw={rtw} nt={nt} splits={splits} depth={depth} n={n}")
     tune = (C.c_int * 7).in_dll(L.lib(), "_ZN2sv11g_gemm_tuneE")
     rng = np.random.default_rng(rtw * 1000 + nt * 100 + splits * 10 + depth + n)
-    m, k = ({1: 384, 2: 512, 4: 768} if nw == 4 else {1: 512, 2: 1024})[rtw], (2560 if splits == 8 else 1280)
+    m, k = {1: 384, 2: 512, 4: 768}[rtw], (2560 if splits == 8 else 1280)
     ws = K.Workspace(16 << 20)
     try:
-        tune[0], tune[1], tune[2], tune[3], tune[4], tune[5], tune[6] = rtw, nt, splits, depth, mf, nw, cpi
+        tune[0], tune[1], tune[2], tune[3], tune[4], tune[5], tune[6] = rtw, nt, splits, depth, 16, 4, 1
         w = torch.from_numpy(rng.normal(0, 0.02, (m, k)).astype(np.float32))
         q, s = quantize_rows(w)
         mi8 = K.matrix(q.cuda(), s.cuda(), 31)
@@ -842,6 +832,45 @@ def test_matmul_gemm_launch_shapes(gpu, shape, n):
                   what=f"bf16 call {call}")
     finally:
         tune[0] = tune[1] = tune[2] = tune[3] = tune[4] = tune[5] = tune[6] = 0
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4, 8])
+@pytest.mark.parametrize("n", [17, 100, 170])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_matmul_gemm32(gpu, splits, n, tiled):
+    """mm_gemm32 (int8 with a scale per row, 256 x 32 blocks of 32-wide tiles) with one to eight k
+    splits of odd and even chunk counts: EPI_NORM with gathered rows and the inverse norms, row-major
+    and tiled, over ragged token blocks; two calls share one workspace."""
+    banner(f"gemm32 splits={splits} n={n} tiled={tiled}")
+    tune = (C.c_int * 7).in_dll(L.lib(), "_ZN2sv11g_gemm_tuneE")
+    rng = np.random.default_rng(splits * 10 + n)
+    m, k = 768, 2560 if splits == 8 else 1280  # 20 chunks in 1, 2 or 4 splits; five in each of 8
+    ws = K.Workspace(16 << 20)
+    w = torch.from_numpy(rng.normal(0, 0.02, (m, k)).astype(np.float32))
+    q, s = quantize_rows(w)
+    mat = K.matrix(q.cuda(), s.cuda(), 31)
+    if tiled:
+        mat = mat.tiled()
+    try:
+        for i, v in enumerate((1, 1, splits, 4, 32, 8, 1)):
+            tune[i] = v
+        for call in range(2):
+            x = (rng.normal(0, 1, (n + 3, k)) * rng.uniform(0.5, 4, (n + 3, 1))).astype(np.float32)
+            rows = rng.permutation(n + 3)[:n].astype(np.uint32)
+            a = L.MatArgs(n, k, m, L.EPI_NORM, L.FLAG_WRITE_INV, m, 0.75, 0, 0, 1, k, 31)
+            aux_ref = np.zeros(n, np.float32)
+            ref = oracle.matmul(L, q.numpy(), s.view(torch.int16).numpy().view(np.uint16), 31, x, a, aux=aux_ref,
+                                x_rows=rows)
+            y = torch.zeros(n, m, device="cuda")
+            aux = torch.zeros(n, device="cuda")
+            K.matmul(mat, to_dev(x), y, n=n, epi=L.EPI_NORM, flags=L.FLAG_WRITE_INV, scale=0.75, aux=aux,
+                     x_rows=to_dev(rows), ws=ws)
+            torch.cuda.synchronize()
+            close(y.cpu().numpy(), ref, atol=5e-5 * max(float(np.abs(ref).max()), 1.0), rtol=1e-4, what=f"call {call}")
+            close(aux.cpu().numpy(), aux_ref, atol=1e-5, rtol=1e-4, what="inv")
+    finally:
+        for i in range(7):
+            tune[i] = 0
 
 
 @pytest.mark.parametrize("rt,nt,cpi", [(1, 1, 2), (1, 2, 2), (1, 4, 1), (2, 1, 1), (2, 2, 1), (2, 4, 1)])
@@ -882,7 +911,7 @@ def test_matmul_pipe_launch_shapes(gpu, rt, nt, cpi, splits, n):
         q, s = quantize_rows(w)
         check(K.matrix(q.cuda(), s.cuda(), 31), q.numpy(), bits(s), 31, L.EPI_NORM, x, "per row",
               L.FLAG_WRITE_INV, rows)
-        for g in (64, 128):
+        for g in (64, 128) if rt == 1 or nt == 1 else ():  # (the larger blocks take no groups)
             q, s = quantize_groups(w, g)
             gs = g.bit_length() - 1
             mat = K.matrix(q.cuda(), s.cuda(), gs)
