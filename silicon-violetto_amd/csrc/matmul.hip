@@ -1132,7 +1132,7 @@ static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
       const uint64_t rounds = (cells * s + 255) / 256;
       const float fill = (float)(cells * s) / (float)(rounds * 256);
       float us = rounds * (5.93f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
-      if (s > 1) us += fill * (c.mf == 32 ? 5.32f + 0.51f * s : (2.51f + 0.98f * s) * (c.rtw * c.nt));
+      if (s > 1) us += fill * (c.mf == 32 ? 5.10f + 0.51f * s : (2.51f + 0.98f * s) * (c.rtw * c.nt));
       offer(c, s, us);
     }
   }
