@@ -339,7 +339,7 @@ def test_attn_verify(gpu, runs_T, p0s, split, tree, rope, allin):
 def test_attn_fused_merge_bit_identical(gpu, runs_T, p0s, split, tree, allin):
     """The merge by the last split to arrive (attention launch only) adds the splits' partials
     in attn_merge_kernel's order (P parts of every P-th split from zero, then the parts in
-    order), so both merges give the same bits: configs[1]'s run (23 splits: four parts; at 33
+    order), so both merges give the same bits: the run of one stream at 8192 keys (23 splits: four parts; at 33
     splits, eight parts, the separate merge runs), ragged runs, a draft tree, 40 runs read from
     memory; both cached-key variants. The second fused call shares the workspace, so it also
     finds the counters back at zero (graph replays rely on it)."""
@@ -377,7 +377,7 @@ def test_attn_fused_merge_bit_identical(gpu, runs_T, p0s, split, tree, allin):
 
 @pytest.mark.parametrize("runs_T,p0s,split", [([5], [65536], 1152), ([5] * 8, [65536] * 8, 3584)])
 def test_attn_verify_long_context(gpu, runs_T, p0s, split):
-    """configs[3]'s attention: 65536 cached keys per stream (1 stream with 1152-key splits, 8
+    """Attention over long contexts: 65536 cached keys per stream (1 stream with 1152-key splits, 8
     streams with 3584-key splits, the engine's choices there), rope on, shuffled pages, the
     variant the launch picks by shape."""
     banner(f"attn long context runs={runs_T} split={split}")
@@ -526,6 +526,30 @@ def test_sample_bit_exact_past_cached(gpu, vocab):
     logits[11, rng.integers(0, vocab, 3)] = np.inf
     logits[12, : vocab - 3] = -np.inf
     rows = sample_rows(n, [0.6, 0.0, 1.0, 0.05, 2.0], [0.95, 0.3, 1.0, 0.05])
+    ref = oracle.sample(L, logits, rows)
+    d_rows = torch.from_numpy(np.frombuffer(bytes((L.SampleRow * n)(*rows)), np.uint8).copy()).cuda()
+    out = torch.zeros(n, dtype=torch.int32, device="cuda")
+    K.sample(to_dev(logits), d_rows, out, None, n, vocab)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().view(np.uint32)
+    assert np.array_equal(got, ref), f"ids differ at rows {np.nonzero(got != ref)[0]}"
+
+
+@pytest.mark.parametrize("vocab", [163840, 163841, 200000])
+def test_sample_bit_exact_past_recorded_batches(gpu, vocab):
+    """Vocabularies at and past the ids whose batch maxima are recorded (32768 + 8 x 16384 = 163840):
+    the later batches are read again in every top-p round. Rows with their likely ids past them,
+    before them and on both sides, one with every id past them masked."""
+    banner(f"sample past recorded batches vocab={vocab}")
+    rng = np.random.default_rng(vocab)
+    n, edge = 24, 163840
+    logits = rng.normal(14.0, 0.6, (n, vocab)).astype(np.float32)
+    for r in range(n):
+        lo, hi = ((min(edge, vocab - 24), vocab), (0, edge), (0, vocab))[r % 3]
+        logits[r, rng.integers(lo, hi, 12)] = rng.uniform(16, 23, 12)
+    logits[8, vocab - 1] = 23.0
+    logits[9, edge:] = -np.inf
+    rows = sample_rows(n, [0.6, 0.0, 1.0, 0.3, 2.0], [0.95, 0.3, 1.0, 0.5])
     ref = oracle.sample(L, logits, rows)
     d_rows = torch.from_numpy(np.frombuffer(bytes((L.SampleRow * n)(*rows)), np.uint8).copy()).cuda()
     out = torch.zeros(n, dtype=torch.int32, device="cuda")
@@ -696,7 +720,7 @@ def test_matmul_many_rows(gpu, m, k, fmt, group, n, epi):
     aux_n = n if epi == L.EPI_NORM else n * m
     # The GPU computes every row; at the largest matrices the oracle checks a seeded sample of
     # 48 rows (each output row depends on its input row alone), so gate_up and down at 512 rows
-    # run in the launch shape the engine uses for configs[4].
+    # run in the launch shape the engine uses for 32 trees of 16 rows.
     rows = np.sort(rng.choice(n, 48, replace=False)).astype(np.uint32) if m * k * n > 2048 * 8192 * 160 else None
     nr = n if rows is None else len(rows)
     a_ref = L.MatArgs(nr, k, m, epi, flags, m - 3, 0.8, 1.1, 0.7, 1, k, gs)
