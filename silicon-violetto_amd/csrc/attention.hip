@@ -57,8 +57,8 @@ constexpr int attn_waves(int D, int, int) { return D == 64 ? 2 : 1; }
 // Whether a run's new keys get a split of their own. All-in-flight variant: yes (it runs beside
 // the cached splits on an otherwise idle CU). Streaming variant up to 32 columns per kv head:
 // no, the last cached split takes them (a split of new keys alone is a short workgroup that
-// holds a resident slot and pushes cached splits into a later round: configs[2] attention 3 %
-// faster). Wider runs: yes (their splits are bound by their own products, and the extra
+// holds a resident slot and pushes cached splits into a later round: attention of 32 streams x 5
+// rows 3 % faster). Wider runs: yes (their splits are bound by their own products, and the extra
 // workgroup adds parallelism: the trees 2 % faster).
 constexpr bool attn_newest_own(int NCT, int NBW) { return NBW > 0 || NCT >= 3; }
 
@@ -88,11 +88,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
   // (split, kv head, run) split-major, so every run's first splits go out before any run's later
   // ones, and the workgroups past a run's last split (the grid is sized for the longest context;
   // they exit once the context length is in) come last, into the tail, instead of holding CU
-  // slots between live ones (configs[2]: about half the grid). Within a split the kv head is the
-  // fastest index (the run fastest measured 4 % slower per step at configs[2]). The all-in-flight
+  // slots between live ones (32 streams of uneven contexts: about half the grid). Within a split the kv head is the
+  // fastest index (the run fastest measured 4 % slower per step of 32 streams). The all-in-flight
   // variant (about one workgroup per CU, few past the context) keeps split fastest: an XCD
   // (workgroup id mod 8) reads every kv head of its splits' pages (split-major measured 0.7 %
-  // slower per step at configs[1], each XCD then reading one kv head's slice of every page).
+  // slower per step of one stream at 8192 keys, each XCD then reading one kv head's slice of every page).
   uint32_t s = blockIdx.x, g = blockIdx.y, r = blockIdx.z;
   if constexpr (NBW == 0) {
     const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), per = gridDim.y * gridDim.z;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves(
     // one), or a grid with too few splits for it, is known once p0 is in, in the round trip of
     // the page words: it leaves before requesting K/V or building queries. The all-in-flight
     // variant (about one workgroup per CU, few past the context) does not wait for p0 before
-    // its K/V requests (measured 8 % slower at configs[1] when it did) and checks after.
+    // its K/V requests (measured 8 % slower at one stream of 8192 keys when it did) and checks after.
     if constexpr (NBW == 0) {
       const uint32_t nsplit = attn_nsplit_t<LOCAL>(p, p0);
       if (nsplit > p.max_splits) {

@@ -22,10 +22,11 @@ namespace sv {
 //     per lane, pass through the wave's own LDS words.
 // What bounds it now: at 1000 rows and more the clock, not the schedule: with random operands the
 // chip holds about 1.7 GHz (products alone reach 1.6-1.9 PFLOP/s of the 2.5 they reach on zeros).
-// MI355X, hi + lo counted: gate_up (16384 x 2048) at 2048 rows 213 us, 1.29 PFLOP/s (mm_gemm32:
-// 290 us, 0.95); down (2048 x 8192) 127 us (154); the 1280-wide model's gate_up in groups of 64
-// at 2048 rows 87 us (mm_gemm: 187). Below 300 rows the operands' way from L2 (a 256-row block
-// reads X at 4 bytes a value), the pipeline's fill and the split's merge are as large.
+// MI355X, hi + lo counted, both sides timed in turn with the weights cold: gate_up (16384 x 2048) at
+// 2048 rows 219 us, 1.26 PFLOP/s (blocks of 512 x 64 with all waves in one phase: 252, 1.09); down
+// (2048 x 8192) 129 us (155, blocks of 256 x 32); the two together 348 (407). The 1280-wide model's
+// gate_up in groups of 64 at 2048 rows 93 us (mm_gemm: 190). Below 300 rows the operands' way from L2
+// (a 256-row block reads X at 4 bytes a value), the pipeline's fill and the split's merge are as large.
 template <int FMT, int RT, int NT, int CPI, bool GR>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void mm_pipe(MMParams p, uint32_t n_tblk) {
   constexpr int BN = 32 * NT, D = RT * NT >= 8 ? 1 : 2;

@@ -42,7 +42,7 @@ class ModelShape:
         return self.n_layers * per + 2 * self.vocab * H
 
 
-# BASELINE.json configs[0..4] shapes; REFERENCE_SHAPE is the reference's own model
+# The 2048-wide 1B decoder of the benchmark's workloads; REFERENCE_SHAPE is the reference's own model
 # (engine/src/model.rs:6-18), kept as a second parity shape.
 CONFIG_SHAPE = ModelShape()
 REFERENCE_SHAPE = ModelShape(hidden=1280, n_heads=10, n_kv_heads=2, head_dim=128, ffn=3328, vocab=151680,

@@ -27,12 +27,12 @@ def layer_launches(eng) -> tuple[int, int]:
 
 
 @pytest.mark.parametrize("n_layers,ctxs,rows", [
-    (2, [1000], 5),       # 5 token slots, 2 column tiles (the configs[1] variant)
+    (2, [1000], 5),       # 5 token slots, 2 column tiles (one stream's variant)
     (2, [2500], 1),       # plain decode: 4 token slots, 1 column tile, 21 splits
     (3, [700], 3),
     (2, [300, 900], 4),   # two runs, 8 rows
     (2, [600], 8),        # 8 rows, 32 columns per kv head
-    (16, [8192], 5),      # configs[1]'s depth and context
+    (16, [8192], 5),      # one stream's depth and context
 ])
 def test_layers_kernel_steps(gpu, n_layers, ctxs, rows):
     banner(f"layer kernel steps: {n_layers} layers, contexts {ctxs}, {rows} rows per run")

@@ -1,7 +1,7 @@
-"""End-to-end verify steps on the GPU engine against the oracle engine (BASELINE.json
-configs[0] and smaller variants), through the C ABI.
+"""End-to-end verify steps on the GPU engine against the oracle engine (one layer
+and head, and smaller variants), through the C ABI.
 
-Bar (north star): logits within 2e-2 max-abs / 1e-2 relative; greedy ids equal wherever the
+Bar: logits within 2e-2 max-abs / 1e-2 relative; greedy ids equal wherever the
 oracle's top-1 margin exceeds 2e-2; accepted counts, emitted ids, paths, lengths and page
 tables bit-exact."""
 from __future__ import annotations
@@ -108,7 +108,7 @@ def compare_step(res, ids_r, logits_r, em_r, extra_r, eng, ref, slots, runs=None
 
 
 def test_config0_step(gpu):
-    """one layer + head, 512 cached tokens, k = 4 uniform drafts, greedy, seed 0."""
+    """One layer + head, 512 cached tokens, k = 4 uniform drafts, greedy, seed 0."""
     banner("config0 step")
     shape = ModelShape(n_layers=1)
     model, gm, eng, ref, slots, rng = build_pair(shape, ctx=512, seed=0)
@@ -354,7 +354,7 @@ def resync(eng, ref, slots) -> None:
 
 @pytest.mark.parametrize("top_p", [1.0, 0.9])
 def test_sampled_graph_replay_multi_stream(gpu, top_p):
-    """configs[2]'s path at reduced size: 8 streams (contexts 64-1100, shuffled page tables), T in
+    """The 32-stream path at reduced size: 8 streams (contexts 64-1100, shuffled page tables), T in
     {0.5, 0.7, 1.0, 1.3}, captured once as a HIP graph and replayed, as bench.py times it.
     First a plain sampled decode records each stream's continuation (14 replays of one row per
     stream); then verify steps of k = 4 drafts from the replay drafter over that continuation
@@ -454,7 +454,7 @@ def test_sampled_graph_replay_multi_stream(gpu, top_p):
     eng.close()
 
 
-TREE16 = [None, 0, 0, 0, 0, 1, 1, 2, 2, 3, 3, 4, 4, 5, 6, 7]  # configs[4]'s tree (16 nodes)
+TREE16 = [None, 0, 0, 0, 0, 1, 1, 2, 2, 3, 3, 4, 4, 5, 6, 7]  # the benchmark's tree (16 nodes)
 
 
 def tree_nodes(parents) -> np.ndarray:
@@ -467,7 +467,7 @@ def tree_nodes(parents) -> np.ndarray:
 
 
 def test_sampled_tree_step_accepts_planted_path(gpu):
-    """Four streams verify configs[4]'s 16-node tree at T = 0.7 (top-p 1 and 0.9) through
+    """Four streams verify the benchmark's 16-node tree at T = 0.7 (top-p 1 and 0.9) through
     sv_step. The drafts along root -> 2 -> 7 -> 15 are set, level by level, to what the oracle
     samples at their parents, so multi-candidate sample-and-match accepts a path that is not a
     prefix of the rows and kv_compact moves it. Draws, emitted counts, paths, lengths and page
@@ -520,8 +520,8 @@ def test_sampled_tree_step_accepts_planted_path(gpu):
 
 
 def test_trees_32_streams_full_layer(gpu):
-    """configs[4]'s step shape at one layer: 32 streams x the 16-node tree (512 verify rows: the
-    GEMM launch shapes and attention grid configs[4] uses), 4096 cached tokens each on shuffled
+    """The tree step's shape at one layer: 32 streams x the 16-node tree (512 verify rows: the
+    GEMM launch shapes and attention grid that step uses), 4096 cached tokens each on shuffled
     pages, random node ids, T = 0.7 sample-and-match, compaction where a path is accepted.
     Draws (CDF-edge rows counted), emitted counts, paths, lengths and page tables against the
     oracle; logits within 2e-2 / 1e-2."""
@@ -748,11 +748,11 @@ def test_prompt_chunks_then_verify(gpu):
 
 @pytest.mark.parametrize("n_seqs", [1, 8])
 def test_config3_long_context_bf16(gpu, n_seqs):
-    """configs[3] end to end: unquantised bf16 weights (N(0, 0.02)) over two layers, 1 or 8
+    """Long contexts end to end: unquantised bf16 weights (N(0, 0.02)) over two layers, 1 or 8
     streams each with 65536 cached tokens (random bf16 K/V), two greedy verify steps of k = 4
     linear drafts, the split-KV attention at the engine's own split choice, against the oracle
     engine: logits, greedy ids, emitted counts, lengths and page tables at the step bar."""
-    banner(f"configs[3] end to end, {n_seqs} stream(s) x 65536")
+    banner(f"long context end to end, {n_seqs} stream(s) x 65536")
     shape = ModelShape(n_layers=2)
     model, gm, eng, ref, slots, rng = build_pair(shape, ctx=65536, n_seqs=n_seqs, seed=31, int8=False,
                                                  max_seq_len=65536 + 64, fast_kv=True, max_head_rows=16 * n_seqs)

@@ -53,7 +53,7 @@ def _call(case, runs_T, p0s, split, noalloc):
 
 @pytest.mark.gpu
 def test_noalloc_matches_allocating_entry_point(gpu):
-    """configs[2]-like first call (32 runs of 5 rows, contexts 1024-8192, 1152-key splits), then a
+    """A serving-like first call (32 runs of 5 rows, contexts 1024-8192, 1152-key splits), then a
     smaller one (3 runs, one with a 16-node tree, 256-key splits): outputs and the new K/V rows
     equal the allocating entry point's bit for bit."""
     rng = np.random.default_rng(5)
