@@ -208,7 +208,8 @@ sv_status sv_rmsnorm_rows(void* stream, const float* d_in, const uint32_t* d_row
  * is chosen from n (the reference's Matmul::for_tokens, encode.rs:33-44). The workspace
  * (sv_matmul_workspace_bytes; zero bytes needs none) carries split-k partials: zero-fill it
  * once; the kernels leave its counters at zero, so calls in stream order may share one, and
- * calls that overlap in time must not. */
+ * calls that overlap in time must not. The size does not grow with n alone (fewer rows may be
+ * split more): a workspace that serves several n is as large as the largest of their sizes. */
 size_t sv_matmul_workspace_bytes(uint32_t n, uint32_t m, uint32_t k);
 sv_status sv_matmul(void* stream, const sv_matrix* w, const float* d_x, const uint32_t* d_x_rows, float* d_y,
                     const float* d_base, float* d_aux, const sv_mat_args* a, void* d_workspace,
