@@ -1086,27 +1086,29 @@ int g_gemm_order = -1;  // tests: force a work order (-1: the modelled choice)
 //    hold two sets of sums with scale groups, and spill: not offered there.
 //  - mm_gemm's blocks of 64 and 80 tokens (bf16 only: there are no conversions to hide) run two a compute
 //    unit, 512 a round: lo up to 256 of them, hi as soon as some unit has two (the bf16 head, 32000 x
-//    2048, at 192 rows: 375 blocks of 64 tokens 79 us, mm_pipe's 250 blocks of 128 tokens 68).
+//    2048, at 192 rows: 375 blocks of 64 tokens 79 us, mm_pipe's 250 blocks of 128 tokens 68); a full
+//    round overlaps the next (0.95).
 //  - mm_gemm's splits of 32-token blocks (128 rows in two with bf16, 64 rows in two to eight with scale
 //    groups): a time linear in blocks and chunks while one round holds them all, three blocks a compute
 //    unit, four with groups (bf16 qkv, 3072 x 2048: 768 blocks at 512 rows 26 us, 816 at 513 rows 28).
 //    They win where the 32-wide blocks are few (qkv at 352 rows 22 us against 25; gate_up in groups at 32
 //    rows 20 against 24).
 // Fitted on MI355X to 7400 launches at 17-2048 rows of the 2048- and 1280-wide models' matrices and
-// heads with their own epilogues, weights cold: over 674 (matrix, format, rows) the choice is 2.0 %
-// slower on average than the fastest of all launches measured, and 4 % at most slower than the better
-// one of the two rules that it replaced (at 6 points more than 3 %).
+// heads with their own epilogues, weights cold, where launches within 5 % of each other are ordered as
+// they were inside whole layers (weights warm): over 674 (matrix, format, rows) the choice is 2.2 % slower
+// on average than the fastest of all launches measured, and 5 % at most slower than the better one of two
+// earlier forms of this rule (at 7 points more than 3 %).
 static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, uint32_t k) {
   static const struct {
     GemmCfg c;
     float lo, hi;  // us per chunk
-  } SHAPES[] = {{{1, 1, 1, 4, 32, 8, 1}, 0.44f, 0.55f}, {{1, 1, 1, 4, 33, 8, 2}, 0.49f, 0.67f},
-                {{1, 2, 1, 4, 33, 8, 2}, 0.77f, 0.95f}, {{2, 1, 1, 4, 33, 8, 1}, 0.98f, 1.07f},
-                {{1, 4, 1, 4, 33, 8, 1}, 1.33f, 1.56f}, {{2, 2, 1, 4, 33, 8, 1}, 1.32f, 1.54f},
-                {{2, 4, 1, 4, 33, 8, 1}, 2.23f, 3.03f}, {{4, 4, 1, 2, 16, 4, 1}, 1.28f, 1.77f},
-                {{2, 5, 1, 2, 16, 4, 1}, 1.12f, 1.41f}};
+  } SHAPES[] = {{{1, 1, 1, 4, 32, 8, 1}, 0.46f, 0.55f}, {{1, 1, 1, 4, 33, 8, 2}, 0.56f, 0.65f},
+                {{1, 2, 1, 4, 33, 8, 2}, 0.82f, 0.93f}, {{2, 1, 1, 4, 33, 8, 1}, 0.99f, 1.18f},
+                {{1, 4, 1, 4, 33, 8, 1}, 1.33f, 1.73f}, {{2, 2, 1, 4, 33, 8, 1}, 1.33f, 1.47f},
+                {{2, 4, 1, 4, 33, 8, 1}, 2.52f, 3.00f}, {{4, 4, 1, 2, 16, 4, 1}, 1.21f, 1.84f},
+                {{2, 5, 1, 2, 16, 4, 1}, 1.09f, 1.50f}};
   const uint32_t nch = k / GKC;
-  const float pipe = grouped ? 1.28f : fmt == SV_FMT_BF16 ? 1.06f : 1.0f;  // mm_pipe's chunks by format
+  const float pipe = grouped ? 1.16f : fmt == SV_FMT_BF16 ? 0.99f : 1.0f;  // mm_pipe's chunks by format
   GemmCfg best{1, 1, 1, 4, 33, 8, 2};
   float best_us = 1e30f;
   auto offer = [&](GemmCfg c, int s, float us) {
@@ -1120,8 +1122,8 @@ static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
     if (c.mf == 16) {
       if (fmt != SV_FMT_BF16) continue;
       const uint64_t rem = cells % 512;
-      float us = cells / 512 * (3.55f + nch * sh.hi);
-      if (rem) us += 3.55f + nch * (rem <= 256 ? sh.lo : sh.hi);
+      float us = cells / 512 * (4.29f + nch * 0.95f * sh.hi);
+      if (rem) us += 4.29f + nch * (rem <= 256 ? sh.lo : sh.hi);
       offer(c, 1, us);
       continue;
     }
@@ -1131,8 +1133,8 @@ static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
       if (s > 1 && (nch % s || nch / s < 4 || cells * s > 256)) continue;
       const uint64_t rounds = (cells * s + 255) / 256;
       const float fill = (float)(cells * s) / (float)(rounds * 256);
-      float us = rounds * (5.93f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
-      if (s > 1) us += fill * (c.mf == 32 ? 5.10f + 0.51f * s : (2.51f + 0.98f * s) * (c.rtw * c.nt));
+      float us = rounds * (5.87f + (nch / s) * (c.mf == 33 ? pipe : 1.0f) * (sh.lo + (sh.hi - sh.lo) * fill * fill));
+      if (s > 1) us += fill * (c.mf == 32 ? 4.96f + 0.36f * s : (2.83f + 1.11f * s) * (c.rtw * c.nt));
       offer(c, s, us);
     }
   }
@@ -1141,7 +1143,7 @@ static GemmCfg pick_by_time(uint32_t fmt, bool grouped, uint32_t n, uint32_t m, 
     for (int s : {2, 4, 8}) {
       if ((s > 2 && !grouped) || nch % s || nch / s < 4 || cells_of(c) * s > (grouped ? 1024u : 768u)) continue;
       const float x = cells_of(c) * s / 512.0f, ch = (float)(nch / s);
-      offer(c, s, grouped ? 0.04f + 0.82f * ch + x * (2.28f + 0.40f * ch) : -0.20f + 0.60f * ch + x * (4.82f + 0.36f * ch));
+      offer(c, s, grouped ? -0.04f + 0.70f * ch + x * (3.29f + 0.41f * ch) : 0.05f + 0.38f * ch + x * (4.55f + 0.52f * ch));
     }
   }
   return best;
